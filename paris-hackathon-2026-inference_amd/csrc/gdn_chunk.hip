@@ -818,12 +818,6 @@ __device__ __forceinline__ void read_rows(RowOps &op, const u32x4 *st, int q, in
   }
 }
 
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
 __device__ __forceinline__ u32x2 pack4(f32x4 x) {
   bf16x4 r;

@@ -147,6 +147,14 @@ __device__ __forceinline__ void gates_from_raw(const GateArgs &ga, const GateRaw
   }
 }
 
+// A workgroup barrier that orders LDS accesses only: outstanding global loads
+// and stores stay in flight across it.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // Sum over the 16 lanes of a DPP row (every lane receives the sum).
 template <int CTRL>
 __device__ __forceinline__ float dpp_mov(float v) {

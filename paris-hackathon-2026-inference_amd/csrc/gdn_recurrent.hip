@@ -1,6 +1,8 @@
-// Token recurrence of the gated delta rule (decode / spec-verify / small-T).
+// Token recurrence of the gated delta rule: recurrent_kernel (decode,
+// spec-verify, short steps) and recurrent_tokens_kernel (sequences of many
+// tokens, below).
 //
-// One workgroup owns a [KD x VT] column slice of one (sequence, v-head)
+// recurrent_kernel: one workgroup owns a [KD x VT] column slice of one (sequence, v-head)
 // state (KD = 128 by default; 64 and 256 are also built, and any v head dim
 // that is a multiple of VT) and keeps it in registers for all of the
 // sequence's tokens: the
@@ -22,6 +24,7 @@ namespace gdn {
 namespace {
 
 typedef __attribute__((ext_vector_type(4))) float f32x4;
+typedef __attribute__((ext_vector_type(2))) float f32x2;
 typedef __attribute__((ext_vector_type(4))) unsigned u32x4;
 
 constexpr int KD_DEFAULT = 128;  // head dim of k (rows of the state) of the tuned build
@@ -314,11 +317,367 @@ __global__ __launch_bounds__(NT) void recurrent_kernel(RecArgs a) {
   }
 }
 
+// ------------------------------------------------------------ token blocks
+// The same recurrence for sequences of many tokens (prefills in fp32 or fp16,
+// or at head dims the chunk kernels are not built for).  recurrent_kernel's
+// token step is a chain of memory and LDS round trips (the next token's inputs
+// are waited for at each barrier, three wave sums go through LDS): 2.3 us per
+// token whatever the batch.  Here a workgroup of 4 waves
+//   * takes TB tokens at a time: their q and k rows, normalised and scaled,
+//     their v columns and gates go into LDS once per block (the next block's
+//     are requested into registers first), so a token step waits on no memory;
+//   * holds few state elements per lane: LPC lanes share a column, lane r of
+//     them owning rows 4 r + e + 4 LPC i (e < 4), CPL columns each, so that a
+//     step is K / LPC * CPL * 4 multiply-adds per lane, the two K-reductions end
+//     on DPP within the LPC lanes, and the outputs wait in LDS for the block's
+//     end.
+// Two tokens run together (step2), so that the chain from one pair to the next
+// holds one reduction.  With 16 lanes per column and one column per lane a
+// pair is about 100 vector instructions, one sequence of 32 v-heads has
+// one wave on every SIMD, and the next pair's operands are read ahead; larger
+// batches (several waves per SIMD) take 8 lanes and read nothing ahead.
+// Bound: the vector ALUs' issue (one wave alone issues about every 9 cycles,
+// two or more waves of a SIMD together about every 5).  Measured, fp32, 32
+// v-heads of 128 x 128, from graphs, against recurrent_kernel: T = 256 at
+// B = 1 / 4 / 8 55.7 / 98.2 / 171.9 against 598 / 624 / 648 us; T = 1024 at
+// B = 1 208 against 2380.
+constexpr int TOK_NT = 256;
+
+// Sum over the LPC (8 or 16) lanes that share a column, in every lane.
+template <int LPC>
+__device__ __forceinline__ float col_sum(float x) {
+  x += dpp_mov<0xB1>(x);                            // quad_perm [1,0,3,2]
+  x += dpp_mov<0x4E>(x);                            // quad_perm [2,3,0,1]
+  x += dpp_mov<0x141>(x);                           // row_half_mirror
+  if constexpr (LPC == 16) x += dpp_mov<0x140>(x);  // row_mirror
+  return x;
+}
+
+// ES: bytes of a q/k/v element (2 or 4); KD: k head dim; LPC, CPL: lanes per
+// column, columns per lane
+template <int ES, int KD, int LPC, int CPL>
+__global__ __launch_bounds__(TOK_NT) void recurrent_tokens_kernel(RecArgs a) {
+  constexpr bool AHEAD = LPC == 16 && KD <= 128 && CPL == 1;
+  constexpr int TB = 4096 / KD;              // tokens per block
+  constexpr int COLS = TOK_NT / LPC * CPL;   // state columns per workgroup
+  constexpr int RPL = KD / LPC;              // state rows per lane
+  constexpr int NI = RPL / 4;                // groups of 4 rows per lane
+  constexpr int PER = KD / 16;               // q and k elements per lane of a row's 16 lanes
+  constexpr int ROWS = TOK_NT / 16;          // q / k rows loaded per pass
+  constexpr int NP = TB / ROWS;              // passes
+  constexpr int VW = PER * ES / 4;           // 32-bit words of one lane's share of a row
+  constexpr int VPT = TB * COLS / TOK_NT;    // v (and o) elements per thread
+  __shared__ __align__(16) float kt[TB][KD], qt[TB][KD];
+  __shared__ __align__(16) float gt[TB][4];  // e^g, beta, q~ . k~, beta e^g (written by two threads: a vector's elements would be stored as one)
+  __shared__ __align__(8) float pt[TB][2];                 // odd tokens: k~ . (the even one before it)'s k~, q~ . that k~
+  __shared__ __align__(16) float vt[TB][COLS], ot[TB][COLS];
+
+  const int tid = threadIdx.x;
+  const int r = tid & (LPC - 1);         // lane within the column
+  const int cb = (tid / LPC) * CPL;      // this lane's first column within the workgroup's
+  const int tiles = a.V / COLS;
+  const int ratio = a.Hv / a.Hk;
+  // the workgroups that read one (sequence, k-head)'s rows on one XCD (workgroups
+  // are dealt to the 8 XCDs in turn)
+  int n, h, tile;
+  {
+    const int per = ratio * tiles;
+    int g = blockIdx.x / per, m = blockIdx.x % per;
+    if ((a.n_seqs * a.Hk) % 8 == 0) {
+      const int t = blockIdx.x >> 3;
+      g = 8 * (t / per) + (blockIdx.x & 7);
+      m = t % per;
+    }
+    n = g / a.Hk;
+    h = (g % a.Hk) * ratio + m / tiles;
+    tile = m % tiles;
+  }
+  const int hk = h / ratio;
+  const int col0 = tile * COLS;
+
+  int64_t t0;
+  int len;
+  seq_range(a.cu, n, a.T, a.total, &t0, &len);
+  len = __builtin_amdgcn_readfirstlane(len);
+
+  // ---- one block's inputs in registers
+  const int row = tid >> 4, l16 = tid & 15;  // the q / k row of pass 0, and the lane's share of it
+  uint32_t qu[NP][VW], ku[NP][VW], vu[VPT], gu[2];
+  auto load_block = [&](int b0) {  // tokens b0 .. b0 + TB of the sequence (rows past its end: its last token)
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      const int64_t tok = t0 + min(b0 + row + ROWS * i, len - 1);
+      const char *qp = static_cast<const char *>(a.q) + (tok * a.qs + (int64_t)hk * KD + l16 * PER) * ES;
+      const char *kp = static_cast<const char *>(a.k) + (tok * a.ks + (int64_t)hk * KD + l16 * PER) * ES;
+      if constexpr (VW % 4 == 0) {
+#pragma unroll
+        for (int w = 0; w < VW; w += 4) {
+          const u32x4 x = *reinterpret_cast<const u32x4 *>(qp + 4 * w), y = *reinterpret_cast<const u32x4 *>(kp + 4 * w);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) qu[i][w + e] = x[e], ku[i][w + e] = y[e];
+        }
+      } else {  // (K = 64 in 2-byte types: 8 bytes)
+        typedef __attribute__((ext_vector_type(2))) unsigned u32x2;
+        const u32x2 x = *reinterpret_cast<const u32x2 *>(qp), y = *reinterpret_cast<const u32x2 *>(kp);
+        qu[i][0] = x.x, qu[i][1] = x.y, ku[i][0] = y.x, ku[i][1] = y.y;
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < VPT; ++i) {
+      const int e = tid + TOK_NT * i;
+      const int64_t tok = t0 + min(b0 + e / COLS, len - 1);
+      vu[i] = load_bits(a.v, tok * a.vs + (int64_t)h * a.V + col0 + e % COLS, a.qkv_dt);
+    }
+    if (tid < TB) {
+      const int64_t gi = (t0 + min(b0 + tid, len - 1)) * a.gate.stride + h;
+      gu[0] = load_bits(a.gate.g_or_a, gi, a.gate.A_log ? a.gate.dt : GDN_DTYPE_F32);
+      gu[1] = load_bits(a.gate.beta_or_b, gi, a.gate.dt);
+    }
+  };
+  const float a_log = a.gate.A_log ? a.gate.A_log[h] : 0.f, dt_bias = a.gate.A_log ? a.gate.dt_bias[h] : 0.f;
+  // ... and from them the block's operands in LDS
+  auto elem = [&](const uint32_t (&u)[VW], int i) -> float {
+    if constexpr (ES == 4)
+      return __uint_as_float(u[i]);
+    else
+      return bits_to_f32((u[i / 2] >> (16 * (i & 1))) & 0xffffu, a.qkv_dt);
+  };
+  auto store_block = [&]() {
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      const int t = row + ROWS * i;
+      float qf[PER], kf[PER], sqq = 0.f, skk = 0.f, sqk = 0.f;
+#pragma unroll
+      for (int e = 0; e < PER; ++e) {
+        qf[e] = elem(qu[i], e);
+        kf[e] = elem(ku[i], e);
+        sqq += qf[e] * qf[e];
+        skk += kf[e] * kf[e];
+        sqk += qf[e] * kf[e];
+      }
+      sqq = row16_sum(sqq);
+      skk = row16_sum(skk);
+      sqk = row16_sum(sqk);
+      const float rq = (a.l2norm ? rsqrtf(sqq + 1e-6f) : 1.f) * a.scale;
+      const float rk = a.l2norm ? rsqrtf(skk + 1e-6f) : 1.f;
+#pragma unroll
+      for (int e = 0; e < PER; e += 4) {
+        *reinterpret_cast<f32x4 *>(&qt[t][l16 * PER + e]) = f32x4{qf[e], qf[e + 1], qf[e + 2], qf[e + 3]} * rq;
+        *reinterpret_cast<f32x4 *>(&kt[t][l16 * PER + e]) = f32x4{kf[e], kf[e + 1], kf[e + 2], kf[e + 3]} * rk;
+      }
+      if (l16 == 0) gt[t][2] = sqk * rq * rk;
+      // (token t - 1 sits in the 16 lanes before these; ROWS is even)
+      float pkk = 0.f, pqk = 0.f;
+      const float rkp = __shfl_xor(rk, 16, 64);
+#pragma unroll
+      for (int e = 0; e < PER; ++e) {
+        const float kp = __shfl_xor(kf[e], 16, 64);
+        pkk += kf[e] * kp;
+        pqk += qf[e] * kp;
+      }
+      pkk = row16_sum(pkk) * rk * rkp;
+      pqk = row16_sum(pqk) * rq * rkp;
+      if (l16 == 0 && (t & 1)) {
+        pt[t][0] = pkk;
+        pt[t][1] = pqk;
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < VPT; ++i) {
+      const int e = tid + TOK_NT * i;
+      vt[e / COLS][e % COLS] = bits_to_f32(vu[i], a.qkv_dt);
+    }
+    if (tid < TB) {
+      float gl, bt;
+      gates_from_raw(a.gate, GateRaw{gu[0], gu[1], a_log, dt_bias}, &gl, &bt);
+      const float eg = expf(gl);
+      gt[tid][0] = eg;
+      gt[tid][1] = bt;
+      gt[tid][3] = bt * eg;
+    }
+  };
+
+  if (len > 0) load_block(0);
+  int64_t in_row = a.state_in ? pool_row_first(a.in_idx, n, a.in_rows) : -1;
+  int64_t out_row = a.state_out ? pool_row_first(a.out_idx, n, a.out_rows) : -1;
+  const int64_t soff = (int64_t)4 * r * a.V + col0 + cb;  // of this lane's row 0, column 0, within a head's state
+  float s[RPL][CPL];
+#pragma unroll
+  for (int j = 0; j < RPL; ++j)
+#pragma unroll
+    for (int c = 0; c < CPL; ++c)
+      s[j][c] = in_row >= 0 ? a.state_in[(in_row * a.Hv + h) * ((int64_t)KD * a.V) + soff +
+                                         (int64_t)(j % 4 + 4 * LPC * (j / 4)) * a.V + c]
+                            : 0.f;
+
+  struct Tok {  // one token's operands of a lane
+    f32x4 k[NI], q[NI];
+    float v[CPL];
+    f32x4 g;
+  };
+  auto read_tok = [&](Tok &x, int t) {
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      x.k[i] = *reinterpret_cast<const f32x4 *>(&kt[t][4 * r + 4 * LPC * i]);
+      x.q[i] = *reinterpret_cast<const f32x4 *>(&qt[t][4 * r + 4 * LPC * i]);
+    }
+#pragma unroll
+    for (int c = 0; c < CPL; ++c) x.v[c] = vt[t][cb + c];
+    x.g = *reinterpret_cast<const f32x4 *>(gt[t]);
+  };
+  // k~^T S and q~^T S of one token over the whole column
+  auto reduce = [&](const Tok &x, float (&pk)[CPL], float (&pq)[CPL]) {
+#pragma unroll
+    for (int c = 0; c < CPL; ++c) pk[c] = pq[c] = 0.f;
+#pragma unroll
+    for (int j = 0; j < RPL; ++j)
+#pragma unroll
+      for (int c = 0; c < CPL; ++c) {
+        pk[c] = __builtin_fmaf(x.k[j / 4][j % 4], s[j][c], pk[c]);
+        pq[c] = __builtin_fmaf(x.q[j / 4][j % 4], s[j][c], pq[c]);
+      }
+#pragma unroll
+    for (int c = 0; c < CPL; ++c) {
+      pk[c] = col_sum<LPC>(pk[c]);
+      pq[c] = col_sum<LPC>(pq[c]);
+    }
+  };
+  // Tokens t and t + 1 together: both reductions run over the state before
+  // them, and token t's rank-1 update enters token t + 1's sums through the
+  // dot products with k~_t, so the chain from one pair to the next holds one
+  // reduction and the state is scaled once.
+  auto step2 = [&](const Tok &x, const Tok &y, f32x2 yx, int t) {
+    float pk0[CPL], pq0[CPL], pk1[CPL], pq1[CPL], d0[CPL], d1[CPL];
+    reduce(x, pk0, pq0);
+    reduce(y, pk1, pq1);
+    const float e01 = x.g.x * y.g.x;
+#pragma unroll
+    for (int c = 0; c < CPL; ++c) {
+      d0[c] = __builtin_fmaf(-x.g.w, pk0[c], x.g.y * x.v[c]);
+      const float sk = __builtin_fmaf(yx.x, d0[c], x.g.x * pk1[c]);  // k~_{t+1}^T S after token t
+      const float sq = __builtin_fmaf(yx.y, d0[c], x.g.x * pq1[c]);
+      d1[c] = __builtin_fmaf(-y.g.w, sk, y.g.y * y.v[c]);
+      if (r == 0) {
+        ot[t][cb + c] = x.g.x * pq0[c] + x.g.z * d0[c];
+        ot[t + 1][cb + c] = y.g.x * sq + y.g.z * d1[c];
+      }
+      d0[c] *= y.g.x;
+    }
+#pragma unroll
+    for (int j = 0; j < RPL; ++j)
+#pragma unroll
+      for (int c = 0; c < CPL; ++c)
+        s[j][c] = __builtin_fmaf(y.k[j / 4][j % 4], d1[c], __builtin_fmaf(x.k[j / 4][j % 4], d0[c], e01 * s[j][c]));
+  };
+  auto step1 = [&](const Tok &x, int t) {
+    float pk[CPL], pq[CPL], d[CPL];
+    reduce(x, pk, pq);
+#pragma unroll
+    for (int c = 0; c < CPL; ++c) {
+      d[c] = __builtin_fmaf(-x.g.w, pk[c], x.g.y * x.v[c]);
+      if (r == 0) ot[t][cb + c] = x.g.x * pq[c] + x.g.z * d[c];
+    }
+#pragma unroll
+    for (int j = 0; j < RPL; ++j)
+#pragma unroll
+      for (int c = 0; c < CPL; ++c) s[j][c] = __builtin_fmaf(x.k[j / 4][j % 4], d[c], x.g.x * s[j][c]);
+  };
+
+  for (int b0 = 0; b0 < len; b0 += TB) {
+    const int nb = min(TB, len - b0);
+    store_block();
+    __syncthreads();
+    if (b0 + TB < len) load_block(b0 + TB);
+    const int pairs = nb >> 1;
+    Tok x0, x1, y0, y1;
+    f32x2 p0, p1;
+    auto read_pair = [&](Tok &x, Tok &y, f32x2 &yx, int t) {
+      read_tok(x, t);
+      read_tok(y, t + 1);
+      yx = *reinterpret_cast<const f32x2 *>(pt[t + 1]);
+    };
+    if constexpr (AHEAD) {  // the next pair's operands are read while a pair runs (at the end: the last one again, unused)
+      if (pairs > 0) read_pair(x0, y0, p0, 0);
+      for (int i = 0; i < pairs; i += 2) {
+        read_pair(x1, y1, p1, 2 * min(i + 1, pairs - 1));
+        step2(x0, y0, p0, 2 * i);
+        if (i + 1 < pairs) {
+          read_pair(x0, y0, p0, 2 * min(i + 2, pairs - 1));
+          step2(x1, y1, p1, 2 * i + 2);
+        }
+      }
+    } else {
+      for (int i = 0; i < pairs; ++i) {
+        read_pair(x0, y0, p0, 2 * i);
+        step2(x0, y0, p0, 2 * i);
+      }
+    }
+    if (nb & 1) {
+      read_tok(x0, nb - 1);
+      step1(x0, nb - 1);
+    }
+    lds_barrier();  // the block's outputs are in LDS, its operands read
+#pragma unroll
+    for (int i = 0; i < VPT; ++i) {
+      const int e = tid + TOK_NT * i;
+      if (e / COLS < nb)
+        store_elem(a.o, ((t0 + b0 + e / COLS) * a.Hv + h) * (int64_t)a.V + col0 + e % COLS, a.o_dt, ot[e / COLS][e % COLS]);
+    }
+  }
+
+  if (out_row >= 0) {
+    float *dst = a.state_out + (out_row * a.Hv + h) * ((int64_t)KD * a.V) + soff;
+#pragma unroll
+    for (int j = 0; j < RPL; ++j)
+#pragma unroll
+      for (int c = 0; c < CPL; ++c) dst[(int64_t)(j % 4 + 4 * LPC * (j / 4)) * a.V + c] = s[j][c];
+  }
+}
+
 }  // namespace
 }  // namespace gdn
 
 namespace gdn {
 namespace {
+
+// Tokens per sequence (their average, with cu_seqlens) from which a call
+// without snapshots takes recurrent_tokens_kernel.  Its token steps are much
+// cheaper, its state accesses less contiguous (16 or 32 columns of a row per
+// workgroup).  Measured from graphs, fp32, 32 v-heads of 128 x 128, this kernel
+// against recurrent_kernel: T = 4 at B = 1 / 4 / 8 7 / 10.6 / 15-17 against
+// 12.2 / 13.5 / 15.8 us; T = 8 at B = 8 / 16 / 64 17.4 / 31-34 / 108-125
+// against 27.1 / 32.3 / 97.7; T = 16 at B = 16 / 64 38.6 / 129-146 against
+// 54.3 / 156.
+inline int64_t tokens_min(int64_t pairs) { return pairs <= 128 ? 4 : pairs <= 256 ? 8 : 16; }
+
+// State columns (pairs x V) from which more rows per lane pay: below
+// REC_TOKENS_MID_COLS a wave per SIMD is all there is and the shortest step
+// wins (16 lanes per column, 1 column per lane); then 8 lanes and, for K = 128,
+// from REC_TOKENS_WIDE_COLS 2 columns per lane (fewer reduction steps and LDS
+// reads per element).  fp32, T = 256, 32 v-heads of 128 x 128, (16, 1) / (8, 1)
+// / (8, 2) lanes and columns: B = 1 55.7 / 75.0 / 116.9 us; B = 2 70.5 / 76.1 /
+// 117.4; B = 4 136 / 98 / 124; B = 8 264 / 195 / 172.  K = 64 at B = 8, T = 128:
+// 56 / 41 / 51; K = 256: 236 / 233 with one column per lane, (16, 2) 199.
+constexpr int64_t REC_TOKENS_MID_COLS = 96 * 128;
+constexpr int64_t REC_TOKENS_WIDE_COLS = 192 * 128;
+
+template <int ES, int KD, int LPC, int CPL>
+void launch_tokens_as(const RecArgs &a, hipStream_t st) {
+  const int64_t blocks = static_cast<int64_t>(a.n_seqs) * a.Hv * (a.V / (TOK_NT / LPC * CPL));
+  hipLaunchKernelGGL((recurrent_tokens_kernel<ES, KD, LPC, CPL>), dim3(static_cast<unsigned>(blocks)), dim3(TOK_NT), 0,
+                     st, a);
+}
+template <int ES, int KD>
+void launch_tokens(const RecArgs &a, hipStream_t st) {  // (V is a multiple of 32)
+  const int64_t cols = static_cast<int64_t>(a.n_seqs) * a.Hv * a.V;
+  if constexpr (KD == 256) {
+    if (cols >= REC_TOKENS_WIDE_COLS) return launch_tokens_as<ES, KD, 16, 2>(a, st);
+  } else {
+    if (KD == 128 && cols >= REC_TOKENS_WIDE_COLS && a.V % 64 == 0) return launch_tokens_as<ES, KD, 8, KD / 64>(a, st);
+    if (cols >= REC_TOKENS_MID_COLS) return launch_tokens_as<ES, KD, 8, 1>(a, st);
+  }
+  launch_tokens_as<ES, KD, 16, 1>(a, st);
+}
 
 int recurrent_fwd(const void *q, const void *k, const void *v, int qkv_dtype,
                   int64_t q_stride_t, int64_t k_stride_t, int64_t v_stride_t, const GateArgs &gate,
@@ -355,11 +714,22 @@ int recurrent_fwd(const void *q, const void *k, const void *v, int qkv_dtype,
             state_out, state_out_idx, state_out_rows, o, snapshots, cu_seqlens, n_seqs, T, Hk, Hv, V,
             cu_seqlens ? static_cast<int64_t>(T) : static_cast<int64_t>(n_seqs) * T,
             scale, l2norm_qk, qkv_dtype, o_dtype};
+  const hipStream_t st = static_cast<hipStream_t>(stream);
+  // q / k rows are read in 16-byte pieces there
+  const int64_t es = static_cast<int64_t>(dtype_size(qkv_dtype));
+  const bool aligned = (reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k)) % 16 == 0 &&
+                       (q_stride_t * es) % 16 == 0 && (k_stride_t * es) % 16 == 0;
+  if (!snapshots && aligned && a.total >= tokens_min(static_cast<int64_t>(n_seqs) * Hv) * n_seqs && n_blocks * 2 <= 0x7fffffff) {
+    if (es == 2)
+      K == 64 ? launch_tokens<2, 64>(a, st) : K == 128 ? launch_tokens<2, 128>(a, st) : launch_tokens<2, 256>(a, st);
+    else
+      K == 64 ? launch_tokens<4, 64>(a, st) : K == 128 ? launch_tokens<4, 128>(a, st) : launch_tokens<4, 256>(a, st);
+    return check_launch(name);
+  }
   const bool capped = n_blocks > REC_CAP_MIN_BLOCKS && (T == 1 || snapshots);
   a.head_major = capped;
   const unsigned lds = !capped ? 0u : T == 1 ? REC_CAP_LDS : REC_SNAP_CAP_LDS;
   const dim3 grid(static_cast<unsigned>(n_blocks)), block(REC_NT);
-  const hipStream_t st = static_cast<hipStream_t>(stream);
   if (K == KD_DEFAULT && V == VD_DEFAULT)
     hipLaunchKernelGGL((recurrent_kernel<REC_VT, REC_NT, KD_DEFAULT, VD_DEFAULT>), grid, block, lds, st, a);
   else if (K == 64)

@@ -302,3 +302,71 @@ def test_repeated_ids_beyond_the_first_64_rows(t):
     assert gdn.state_rel_err(np64(pool_gpu[ids[live].to(DEV)]), s_ref[live]) < S_TOL
     untouched = np.setdiff1d(np.arange(n_slots), ids[live].numpy())
     assert torch.equal(pool_gpu[untouched].cpu(), pool[untouched])
+
+
+# recurrent_tokens_kernel: token-block edges (32 tokens at K = 128, 16 at 256, 64 at 64; odd counts end
+# on a single token), and each lane split of its dispatch (B = 1, 4, 8 at 32 v-heads)
+@pytest.mark.parametrize("b,t,dt,kd,vd", [
+    (1, 4, torch.float32, 128, 128), (1, 33, torch.float16, 128, 128), (1, 97, torch.float32, 128, 128),
+    (4, 32, torch.float32, 128, 128), (4, 35, torch.bfloat16, 128, 96), (8, 16, torch.bfloat16, 128, 128),
+    (8, 65, torch.float32, 128, 128), (1, 17, torch.float16, 256, 64), (8, 31, torch.float32, 256, 64),
+    (2, 129, torch.bfloat16, 64, 160), (8, 64, torch.float32, 64, 128)])
+def test_token_blocks_match_oracle(b, t, dt, kd, vd):
+    hk, hv = 16, 32
+    gen = torch.Generator().manual_seed(100 * b + t)
+    q, k = (torch.randn(b, t, hk, kd, generator=gen).to(dt) for _ in range(2))
+    v = torch.randn(b, t, hv, vd, generator=gen).to(dt)
+    g, beta = -torch.rand(b, t, hv, generator=gen), torch.rand(b, t, hv, generator=gen)
+    h0 = torch.randn(b, hv, kd, vd, generator=gen) * 0.1
+    o_ref, s_ref = gdn.recurrent_gated_delta_rule(*(x.float().numpy() for x in (q, k, v, g, beta)),
+                                                  initial_state=h0.numpy())
+    print(f"B={b} T={t} K={kd} V={vd} {dt}", flush=True)
+    o, s = fused_recurrent_gated_delta_rule(*cuda(q, k, v, g, beta), initial_state=h0.to(DEV),
+                                            output_final_state=True, use_qk_l2norm_in_kernel=True)
+    assert np.abs(np64(o) - o_ref).max() <= (1e-4 if dt == torch.float32 else O_TOL_BF16)
+    assert gdn.state_rel_err(np64(s), s_ref) <= 1e-5
+    # q one element past 16-byte alignment: the general kernel, the same result to fp32 rounding
+    qs = torch.zeros(q.numel() + 8, dtype=dt, device=DEV)
+    qs[1:1 + q.numel()] = q.to(DEV).flatten()
+    from engine.kernels import _lib
+    lib, o2, s2 = _lib.load(), torch.empty_like(o), torch.empty_like(s)
+    kk, vv, gg, bb, hh = cuda(k, v, g, beta, h0)
+    st = lib.gdn_recurrent_fwd(qs.data_ptr() + qs.element_size(), kk.data_ptr(), vv.data_ptr(), _lib.GDN_DTYPE[dt],
+                               hk * kd, hk * kd, hv * vd, gg.data_ptr(), bb.data_ptr(), 0, hh.data_ptr(), None, b,
+                               s2.data_ptr(), None, b, o2.data_ptr(), _lib.GDN_DTYPE[dt], None, None, b, t, hk, hv,
+                               kd, vd, kd ** -0.5, 1, _lib.stream_of(o))
+    _lib.check(st, "gdn_recurrent_fwd")
+    assert np.abs(np64(o2) - o_ref).max() <= (1e-4 if dt == torch.float32 else O_TOL_BF16)
+    assert gdn.state_rel_err(np64(s2), np64(s)) <= 1e-5
+
+
+def test_token_blocks_packed_sequences_on_a_pool():
+    """Packed sequences (empty, one token, odd, longer than a block) on a slot pool in place with a repeated
+    and a negative id: against one call per sequence's oracle; unowned slots keep their bits."""
+    lens, slots, rows, hk, hv = [40, 0, 1, 67, 33, 5], [4, 2, 0, 4, -1, 5], 7, 2, 4
+    cu = torch.tensor([0] + list(np.cumsum(lens)), dtype=torch.int32)
+    gen = torch.Generator().manual_seed(7)
+    t = sum(lens)
+    q, k = (torch.randn(1, t, hk, 128, generator=gen) for _ in range(2))
+    v = torch.randn(1, t, hv, 128, generator=gen)
+    g, beta = -torch.rand(1, t, hv, generator=gen), torch.rand(1, t, hv, generator=gen)
+    pool = torch.randn(rows, hv, 128, 128, generator=gen) * 0.1
+    p = pool.to(DEV)
+    o, _ = fused_recurrent_gated_delta_rule(*cuda(q, k, v, g, beta), initial_state=p, inplace_final_state=True,
+                                            ssm_state_indices=torch.tensor(slots, device=DEV), cu_seqlens=cu.to(DEV),
+                                            use_qk_l2norm_in_kernel=True)
+    seen = set()
+    for n, (ln, sl) in enumerate(zip(lens, slots)):
+        own = sl >= 0 and sl not in seen
+        seen.add(sl)
+        h0 = pool[sl:sl + 1].numpy() if own else np.zeros((1, hv, 128, 128))
+        if ln:
+            a = [x[:, cu[n]:cu[n + 1]].numpy() for x in (q, k, v, g, beta)]
+            o_ref, s_ref = gdn.recurrent_gated_delta_rule(*a, initial_state=h0)
+            assert np.abs(np64(o)[:, cu[n]:cu[n + 1]] - o_ref).max() <= 1e-4, n
+        else:
+            s_ref = h0
+        if own:
+            assert gdn.state_rel_err(np64(p[sl:sl + 1]), s_ref) <= 1e-5, n
+    for sl in set(range(rows)) - set(slots):
+        assert torch.equal(p[sl].cpu(), pool[sl])
