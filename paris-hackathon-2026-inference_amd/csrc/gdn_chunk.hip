@@ -50,7 +50,13 @@
 // indices {4g..4g+3, 16+4g..16+4g+3} ("pi" order); the scan's A-operand
 // blocks are stored in the same order, so an accumulator becomes an operand
 // by conversion to bf16 alone (in the scan, between waves, through LDS
-// without any reordering).
+// without any reordering).  Over positions pi order is taken as it is.  Over
+// the k dims (state rows) the tiles are assigned so that a lane's eight
+// accumulators of a tile pair are eight consecutive dims (key_dim): the q and
+// k rows that meet them are then read 16 bytes at a time, from HBM and from
+// LDS, instead of in two pieces of 8 (with plain tiles and 3 unused blocks
+// staged per chunk: T = 4096 102.8 us against 100.0, B = 8 / 16 x T = 1038
+// 126.9 / 249.7 against 121.5 / 240.7 us).
 #include <algorithm>
 #include <type_traits>
 
@@ -75,7 +81,7 @@ constexpr int SCAL = 256;  // per (chunk, v-head) scalars: sq[64], sk[64], eL (1
 // q and k rows from the inputs themselves.)
 constexpr int NB_W = 16;
 constexpr int NB_A = 8;
-constexpr int NB_SC = SCAL / 64;  // scalars as blocks (1)
+constexpr int NB_SC = SCAL / 256;  // scalars as blocks (1 KiB: 256 floats)
 constexpr int VH_W = 0, VH_A = VH_W + NB_W, VH_SC = VH_A + NB_A, NB_VH = VH_SC + NB_SC;
 
 __device__ __forceinline__ f32x4 mfma(bf16x8 a, bf16x8 b, f32x4 c) {
@@ -221,16 +227,21 @@ __global__ __launch_bounds__(256) void chunk_table_kernel(ChunkArgs a) {
 // ------------------------------------------------------------------ phase A
 // One workgroup of 4 waves per (chunk, v-head); wave p owns chunk rows
 // 16p..16p+15.  Fragment layouts used below (lane = 16 g + r, r < 16):
-//   pi fragment of X (bf16 MFMA operand, k-step s):  lane holds row r of the
-//     tile, columns 32s + 4g + 0..3 and 32s + 16 + 4g + 0..3;
+//   fragment of X's rows (bf16 MFMA operand, k-step s):  lane holds row r of
+//     the tile, dims 32s + 8g + 0..7 (one 16-byte read; frag_row);
+//   pi fragment of X^T (k-step s over positions):  lane holds column r of the
+//     tile, positions 32s + 4g + 0..3 and 32s + 16 + 4g + 0..3;
 //   row layout (16x16 fp32 block):  lane holds X[r][4g + e], e < 4;
 //   D layout (16x16 fp32 block):    lane holds X[4g + e][r] (an MFMA result).
 
-// Row-major [64][128] bf16 tile (K or V): 16-byte segment seg of row r is
-// stored at segment seg ^ (r & 15).  Row writes, pi-fragment reads and the
-// transposing reads below are all free of bank conflicts with it.
+// Row-major [64][128] bf16 tile (K, Q or V): 16-byte segment seg of row r is
+// stored at segment seg ^ row_swizzle(r).  Row writes, fragment reads (16 rows,
+// one segment) and the transposing reads below (4 rows, whose swizzles differ
+// in the upper two bits: 2 or 4 segments each) are free of bank conflicts
+// with it.
+__device__ __forceinline__ int row_swizzle(int row) { return ((row & 3) << 2) | ((row >> 2) & 3); }
 __device__ __forceinline__ int nsw(int row, int col) {
-  return row * DK + ((((col >> 3) ^ row) & 15) << 3) + (col & 7);
+  return row * DK + (((col >> 3) ^ row_swizzle(row)) << 3) + (col & 7);
 }
 
 typedef __attribute__((ext_vector_type(4))) short s16x4;
@@ -253,12 +264,24 @@ __device__ __forceinline__ bf16x8 frag_tr(const uint16_t *tile, int s, int n0, i
   const s16x4 hi = ld_tr(tile, 32 * s + 16 + 4 * g4, n0, lane);
   return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
 }
-// Pi fragment of rows row0..row0+15 of X, k-step s.
-__device__ __forceinline__ bf16x8 frag_pi(const uint16_t *tile, int row0, int s, int lane) {
-  const int r = row0 + (lane & 15), g4 = lane >> 4;
-  const u32x2 a = *reinterpret_cast<const u32x2 *>(tile + nsw(r, 32 * s + 4 * g4));
-  const u32x2 b = *reinterpret_cast<const u32x2 *>(tile + nsw(r, 32 * s + 16 + 4 * g4));
-  return as_bf16x8(u32x4{a.x, a.y, b.x, b.y});
+// The k dims (state rows) of tile t, t < 8: row 4 g + e of the tile is dim
+// key_dim(t, g, e), so that the accumulators of tiles 2 s and 2 s + 1 together hold
+// dims 32 s + 8 g .. + 7 in lane group g.  As an operand they then pair with
+// 16 consecutive bytes of a q or k row (frag_row).
+__device__ __forceinline__ int key_dim(int t, int g4, int e) { return 32 * (t >> 1) + 8 * g4 + 4 * (t & 1) + e; }
+// Pi fragment of K^T for k-step s over the positions and the dims of tile t.
+__device__ __forceinline__ bf16x8 frag_kt(const uint16_t *tile, int s, int t, int lane) {
+  const int g4 = lane >> 4, L = lane & 15, col = key_dim(t, L & 3, 0);
+  const auto at = [&](int j0) {
+    return __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+        (lds_s16x4 *)(const_cast<uint16_t *>(tile) + nsw(j0 + (L >> 2), col)));
+  };
+  const s16x4 lo = at(32 * s + 4 * g4), hi = at(32 * s + 16 + 4 * g4);
+  return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+}
+// Rows row0..row0+15 of X, k-step s: dims 32 s + 8 g .. + 7 of row r.
+__device__ __forceinline__ bf16x8 frag_row(const uint16_t *tile, int row0, int s, int lane) {
+  return as_bf16x8(*reinterpret_cast<const u32x4 *>(tile + nsw(row0 + (lane & 15), 32 * s + 8 * (lane >> 4))));
 }
 
 // 16x16x16 fp32 product on MFMA (v_mfma_f32_16x16x4_f32: lane (r, g) gives
@@ -365,10 +388,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void c
   const int g4 = lane >> 4;
   const int r16 = lane & 15;
   const size_t ch = static_cast<size_t>(jl) * a.Hv + h;
-  const int irow = 16 * p + r16;  // this lane's chunk row in row-layout / pi fragments
+  const int irow = 16 * p + r16;  // this lane's chunk row in row layout / row fragments
 
   // ---- global loads: K, V rows (16 bytes per thread), this wave's Q rows as
-  // pi fragments, and the gates
+  // fragments, and the gates
   const int seg = tid & 15;
   u32x4 ku[4], vu[4];
 #pragma unroll
@@ -381,15 +404,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void c
   }
   bf16x8 qf[4];
   {
-    const uint16_t *qrow = a.q + (t0 + irow) * a.qs + (int64_t)hk * DK + 4 * g4;
+    const uint16_t *qrow = a.q + (t0 + irow) * a.qs + (int64_t)hk * DK + 8 * g4;
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
-      u32x2 x0 = {0u, 0u}, x1 = {0u, 0u};
-      if (irow < len) {
-        x0 = *reinterpret_cast<const u32x2 *>(qrow + 32 * s);
-        x1 = *reinterpret_cast<const u32x2 *>(qrow + 32 * s + 16);
-      }
-      qf[s] = as_bf16x8(u32x4{x0.x, x0.y, x1.x, x1.y});
+      u32x4 x = {0u, 0u, 0u, 0u};
+      if (irow < len) x = *reinterpret_cast<const u32x4 *>(qrow + 32 * s);
+      qf[s] = as_bf16x8(x);
     }
   }
   // an odd v-head with per-v-head q / k (dup): its rows against the even
@@ -403,13 +423,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void c
       const int row = min((tid >> 4) + 16 * it, len - 1);
       kpart[it] = *reinterpret_cast<const u32x4 *>(a.k + (t0 + row) * a.ks + (int64_t)(hk - 1) * DK + seg * 8);
     }
-    const uint16_t *qrow = a.q + (t0 + min(irow, len - 1)) * a.qs + (int64_t)(hk - 1) * DK + 4 * g4;
+    const uint16_t *qrow = a.q + (t0 + min(irow, len - 1)) * a.qs + (int64_t)(hk - 1) * DK + 8 * g4;
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      const u32x2 x0 = *reinterpret_cast<const u32x2 *>(qrow + 32 * s);
-      const u32x2 x1 = *reinterpret_cast<const u32x2 *>(qrow + 32 * s + 16);
-      qpart[s] = u32x4{x0.x, x0.y, x1.x, x1.y};
-    }
+    for (int s = 0; s < 4; ++s) qpart[s] = *reinterpret_cast<const u32x4 *>(qrow + 32 * s);
   }
   GateRaw graw{0u, 0u, 0.f, 0.f};
   if (p == 0 && lane < len) {
@@ -500,9 +516,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void c
   const float gi = gam_s[irow], bi = beta_s[irow], nki = nk_s[irow], nqi = nq_s[irow];
   // (register arrays are only indexed by unrolled loop counters; the wave's
   // own block is selected with uniform branches)
-  bf16x8 kown[4];  // pi fragments of this wave's K rows
+  bf16x8 kown[4];  // fragments of this wave's K rows
 #pragma unroll
-  for (int s = 0; s < 4; ++s) kown[s] = frag_pi(kn, 16 * p, s, lane);
+  for (int s = 0; s < 4; ++s) kown[s] = frag_row(kn, 16 * p, s, lane);
   f32x4 lf[4], af[4];  // L and A blocks (p, cb), row layout
 #pragma unroll
   for (int cb = 0; cb < 4; ++cb) {
@@ -512,7 +528,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void c
       f32x4 kk = {0.f, 0.f, 0.f, 0.f}, qk = kk;
 #pragma unroll
       for (int s = 0; s < 4; ++s) {
-        const bf16x8 kcb = frag_pi(kn, 16 * cb, s, lane);
+        const bf16x8 kcb = frag_row(kn, 16 * cb, s, lane);
         kk = mfma(kcb, kown[s], kk);
         qk = mfma(kcb, qf[s], qk);
       }
@@ -625,7 +641,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void c
       pack_hilo(trow[2 * s] * be0, trow[2 * s + 1] * be1, uhi, ulo);
 #pragma unroll
       for (int nb = 0; nb < 8; ++nb) {
-        const bf16x8 kt = frag_tr(kn, s, 16 * nb, lane);
+        const bf16x8 kt = frag_kt(kn, s, nb, lane);
         const bf16x8 vf = frag_tr(vn, s, 16 * nb, lane);
         wt[nb] = mfma(kt, whi, wt[nb]);
         wt[nb] = mfma(kt, wlo, wt[nb]);
@@ -779,7 +795,7 @@ __device__ __forceinline__ void stage_copy(u32x4 *st, const RowSrc &r, const Chu
       }
     } else {
       const int b = i & 15, row = 4 * b + rl;
-      const int seg = 16 * (ps ^ (row & 15));  // (the whole offset is in the range-checked vector offset)
+      const int seg = 16 * (ps ^ row_swizzle(row));  // (the whole offset is in the range-checked vector offset)
       if (i < 16)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(r.k, st + (RS_K + b) * 64, 16, row * static_cast<int>(a.ks * 2) + seg,
                                                  0, 0, 0);
@@ -801,16 +817,16 @@ __device__ __forceinline__ void read_rows(RowOps &op, const u32x4 *st, int q, in
     op.u = __builtin_bit_cast(f32x4, st[(RS_U + q) * 64 + lane]);
     op.sk = *reinterpret_cast<const f32x4 *>(sc + CK + 16 * q + 4 * (lane >> 4));
     op.eL = sc[2 * CK];
-  } else if constexpr (G == 1) {  // Q S: pi fragments of q rows 16q..
+  } else if constexpr (G == 1) {  // Q S: fragments of q rows 16q..
     const uint16_t *qn = reinterpret_cast<const uint16_t *>(st + RS_Q * 64);
 #pragma unroll
-    for (int s = 0; s < 4; ++s) op.qm[s] = __builtin_bit_cast(u32x4, frag_pi(qn, 16 * q, s, lane));
+    for (int s = 0; s < 4; ++s) op.qm[s] = __builtin_bit_cast(u32x4, frag_row(qn, 16 * q, s, lane));
   } else if constexpr (G == 2) {  // S += K^T V'': K^T tiles 2q + t, read transposed from the k rows
     const uint16_t *kn = reinterpret_cast<const uint16_t *>(st + RS_K * 64);
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
-      for (int s = 0; s < 2; ++s) op.kt[2 * t + s] = __builtin_bit_cast(u32x4, frag_tr(kn, s, 32 * q + 16 * t, lane));
+      for (int s = 0; s < 2; ++s) op.kt[2 * t + s] = __builtin_bit_cast(u32x4, frag_kt(kn, s, 2 * q + t, lane));
   } else {  // the output
     op.am[0] = st[(RS_VH + VH_A + 2 * q) * 64 + lane];
     op.am[1] = st[(RS_VH + VH_A + 2 * q + 1) * 64 + lane];  // (unused for q < 2)
@@ -1000,7 +1016,6 @@ __global__ __launch_bounds__(64 * SCAN_WAVES) void chunk_scan_kernel(ChunkArgs a
   const int64_t in_row = a.h0 ? uniform64(pool_row_first(a.h0_idx, n, a.h0_rows)) : -1;
   const int64_t out_row = a.hT ? uniform64(pool_row_first(a.hT_idx, n, a.hT_rows)) : -1;
   const int64_t kv = static_cast<int64_t>(DK) * DV;
-  const int row0 = 32 * q;  // first state row of a compute wave
   if (cs == ce) {  // empty sequence: the final state is the initial one (handled once)
     if (wave < 4 && a.seg_begin == 0 && out_row >= 0) {
       float *dst = a.hT + (out_row * a.Hv + h) * kv + col;
@@ -1008,7 +1023,7 @@ __global__ __launch_bounds__(64 * SCAN_WAVES) void chunk_scan_kernel(ChunkArgs a
       for (int t = 0; t < 2; ++t)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const int r = row0 + 16 * t + 4 * g4 + e;
+          const int r = key_dim(2 * q + t, g4, e);
           dst[r * DV] = in_row >= 0 ? a.h0[(in_row * a.Hv + h) * kv + r * DV + col] : 0.f;
         }
     }
@@ -1035,13 +1050,13 @@ __global__ __launch_bounds__(64 * SCAN_WAVES) void chunk_scan_kernel(ChunkArgs a
   }
   float *carry = a.carry + (static_cast<int64_t>(n) * a.Hv + h) * kv + col;
 
-  f32x4 S[2];  // state rows row0 + 16t + 4g + e of this lane's column
+  f32x4 S[2];  // tiles 2q, 2q + 1: state rows key_dim(2q + t, g, e) of this lane's column
   const float *src = lo == cs ? (in_row >= 0 ? a.h0 + (in_row * a.Hv + h) * kv + col : nullptr) : carry;
   if (src) {
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) S[t][e] = src[(row0 + 16 * t + 4 * g4 + e) * DV];
+      for (int e = 0; e < 4; ++e) S[t][e] = src[key_dim(2 * q + t, g4, e) * DV];
   } else {
 #pragma unroll
     for (int t = 0; t < 2; ++t) S[t] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -1098,7 +1113,7 @@ __global__ __launch_bounds__(64 * SCAN_WAVES) void chunk_scan_kernel(ChunkArgs a
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) dst[(row0 + 16 * t + 4 * g4 + e) * DV] = S[t][e];
+      for (int e = 0; e < 4; ++e) dst[key_dim(2 * q + t, g4, e) * DV] = S[t][e];
   }
 }
 
@@ -1133,19 +1148,18 @@ __global__ __launch_bounds__(64 * SCAN_WAVES) void chunk_scan_persist_kernel(Chu
   const int hk = h / ratio;
   const int col = 16 * ct + (lane & 15);
   const int64_t kv = static_cast<int64_t>(DK) * DV;
-  const int row0 = 32 * q;
   auto state_at = [&](float *base, int64_t row) { return base + (row * a.Hv + h) * kv + col; };
   auto load_state = [&](const float *src, f32x4 (&S)[2]) {
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) S[t][e] = src ? src[(row0 + 16 * t + 4 * g4 + e) * DV] : 0.f;
+      for (int e = 0; e < 4; ++e) S[t][e] = src ? src[key_dim(2 * q + t, g4, e) * DV] : 0.f;
   };
   auto store_state = [&](float *dst, const f32x4 (&S)[2]) {
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) dst[(row0 + 16 * t + 4 * g4 + e) * DV] = S[t][e];
+      for (int e = 0; e < 4; ++e) dst[key_dim(2 * q + t, g4, e) * DV] = S[t][e];
   };
   auto init_src = [&](int64_t row) -> const float * {
     return row >= 0 ? state_at(const_cast<float *>(a.h0), row) : nullptr;
@@ -1302,7 +1316,7 @@ __global__ __launch_bounds__(64 * SCAN_WAVES) void chunk_scan_persist_kernel(Chu
 // accumulators (pi order), V'' the B operand of the state update, so no
 // product needs another wave's registers.  The chunk operands live in LDS in
 // the layouts their consumers read with one ds_read_b128 per fragment: -W
-// and A blocks as in the workspace layout, q rows as pi fragments (written
+// and A blocks as in the workspace layout, q rows as fragments (written
 // from the prep waves' own fragments), K^T fragments (written by the wave of
 // the prep that reads all of them), U tiles by (column tile, position tile).
 // Same algorithm and precision as prep + scan.
@@ -1319,7 +1333,7 @@ struct LocLds {
   uint16_t *kn;     // [64 * 128] K rows (nsw swizzle)
   f32x4 *s16k;      // [1024]: V rows (nsw) / the solve's exchange buffers
   u32x4 *ktf;       // [16][64] K^T fragments (row tile nb, position k-step s) at 2 nb + s
-  u32x4 *qp;        // [16][64] q pi fragments (position tile i, k-step s) at 4 i + s
+  u32x4 *qp;        // [16][64] q fragments (position tile i, k-step s) at 4 i + s
   u32x4 *wb;        // [16][64] -W blocks (p, s) at 4 p + s
   f32x4 *ub;        // [32][64] U tiles (column tile nb, position tile p) at 4 nb + p
   u32x4 *ab;        // [LOC_NB_A][64] A blocks (p, s) at a_blk(p, s)
@@ -1357,10 +1371,8 @@ __device__ __forceinline__ void loc_load(const ChunkArgs &a, LocIn &in, int64_t 
   if (part == 1) return;
 #pragma unroll
   for (int s = 0; s < 4; ++s) {
-    const int off = irow * qs2 + (32 * s + 4 * g4) * 2;
-    const u32x2 x0 = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rq, off, 0, 0));
-    const u32x2 x1 = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rq, off + 32, 0, 0));
-    in.qf[s] = as_bf16x8(u32x4{x0.x, x0.y, x1.x, x1.y});
+    const int off = irow * qs2 + (32 * s + 8 * g4) * 2;
+    in.qf[s] = as_bf16x8(__builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rq, off, 0, 0)));
   }
 }
 
@@ -1469,7 +1481,7 @@ __device__ __forceinline__ void loc_prep(const ChunkArgs &a, const LocIn &in, co
       if (cb <= pa) {
         f32x4 qk = z4a;
 #pragma unroll
-        for (int s = 0; s < 4; ++s) qk = mfma(frag_pi(kn, 16 * cb, s, lane), qa[s], qk);
+        for (int s = 0; s < 4; ++s) qk = mfma(frag_row(kn, 16 * cb, s, lane), qa[s], qk);
         const f32x4 gj = *reinterpret_cast<const f32x4 *>(L.gam_s + 16 * cb + 4 * g4);
         const f32x4 nj = *reinterpret_cast<const f32x4 *>(L.nk_s + 16 * cb + 4 * g4);
 #pragma unroll
@@ -1485,7 +1497,7 @@ __device__ __forceinline__ void loc_prep(const ChunkArgs &a, const LocIn &in, co
   const float gi = L.gam_s[irow], bi = L.beta_s[irow], nki = L.nk_s[irow];
   bf16x8 kown[4];
 #pragma unroll
-  for (int s = 0; s < 4; ++s) kown[s] = frag_pi(kn, 16 * p, s, lane);
+  for (int s = 0; s < 4; ++s) kown[s] = frag_row(kn, 16 * p, s, lane);
   f32x4 lf[4];
 #pragma unroll
   for (int cb = 0; cb < 4; ++cb) {
@@ -1493,7 +1505,7 @@ __device__ __forceinline__ void loc_prep(const ChunkArgs &a, const LocIn &in, co
     if (cb <= p) {
       f32x4 kk = z4a;
 #pragma unroll
-      for (int s = 0; s < 4; ++s) kk = mfma(frag_pi(kn, 16 * cb, s, lane), kown[s], kk);
+      for (int s = 0; s < 4; ++s) kk = mfma(frag_row(kn, 16 * cb, s, lane), kown[s], kk);
       const f32x4 gj = *reinterpret_cast<const f32x4 *>(L.gam_s + 16 * cb + 4 * g4);
       const f32x4 nj = *reinterpret_cast<const f32x4 *>(L.nk_s + 16 * cb + 4 * g4);
 #pragma unroll
@@ -1563,7 +1575,7 @@ __device__ __forceinline__ void loc_prep(const ChunkArgs &a, const LocIn &in, co
   for (int jn = 0; jn < 2; ++jn)
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
-      kt[jn][s] = frag_tr(kn, s, 16 * (2 * p + jn), lane);
+      kt[jn][s] = frag_kt(kn, s, 2 * p + jn, lane);
       L.ktf[(2 * (2 * p + jn) + s) * 64 + lane] = __builtin_bit_cast(u32x4, kt[jn][s]);
     }
 #pragma unroll
@@ -1723,7 +1735,7 @@ __global__ __launch_bounds__(64 * LOC_WAVES) void chunk_local_kernel(ChunkArgs a
   const int64_t in_row = a.h0 ? uniform64(pool_row_first(a.h0_idx, n, a.h0_rows)) : -1;
   const int64_t out_row = a.hT ? uniform64(pool_row_first(a.hT_idx, n, a.hT_rows)) : -1;
   float *dst[2];
-  f32x4 S[2][8];  // tile j: state rows 16 t + 4 g + e of column 32 cw + 16 j + r
+  f32x4 S[2][8];  // tile t: state rows key_dim(t, g, e) of column 32 cw + 16 j + r
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
     const int col = 32 * cw + 16 * j + r16;
@@ -1732,7 +1744,7 @@ __global__ __launch_bounds__(64 * LOC_WAVES) void chunk_local_kernel(ChunkArgs a
 #pragma unroll
     for (int t = 0; t < 8; ++t)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) S[j][t][e] = src ? src[(16 * t + 4 * g4 + e) * DV] : 0.f;
+      for (int e = 0; e < 4; ++e) S[j][t][e] = src ? src[key_dim(t, g4, e) * DV] : 0.f;
   }
   typedef typename std::conditional<BF16_OUT, uint16_t, float>::type OT;
   const int64_t ostep = static_cast<int64_t>(a.Hv) * DV;
@@ -1851,7 +1863,7 @@ __global__ __launch_bounds__(64 * LOC_WAVES) void chunk_local_kernel(ChunkArgs a
 #pragma unroll
       for (int t = 0; t < 8; ++t)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) dst[j][(16 * t + 4 * g4 + e) * DV] = S[j][t][e];
+        for (int e = 0; e < 4; ++e) dst[j][key_dim(t, g4, e) * DV] = S[j][t][e];
     }
 }
 
