@@ -27,18 +27,19 @@
 //                       1 KiB block per (MFMA, wave), lane l's 16 bytes at
 //                       offset 16 l (the scan reads q and k rows from the
 //                       inputs themselves).
-//   chunk_scan_kernel   one workgroup per (sequence, v-head, 16 state
-//                       columns), serial over the chunks: four compute waves,
+//   chunk_scan_kernel   (up to 32 (sequence, v-head) pairs) one workgroup per
+//                       (sequence, v-head, 16 state columns), serial over the
+//                       chunks: four compute waves,
 //                       each owning 16 chunk positions and 32 state rows (its
 //                       state slice lives in MFMA accumulators for the whole
 //                       sequence), exchange V'' and the state through LDS;
 //                       two loader waves stream the operand blocks of the
 //                       chunk after next into a double-buffered LDS stage
 //                       with buffer_load ... lds.
+//   chunk_scan_cols_kernel  (more pairs) the same with 32 or 64 state columns
+//                       per workgroup, 16 to a compute wave.
 // Inputs longer than one segment (64 chunks) run prep / scan per segment,
-// one segment after the other on the caller's stream; several sequences
-// (varlen or a batch) are scanned by one workgroup per (v-head, 16 state
-// columns) walking all of them (chunk_scan_persist_kernel).
+// one segment after the other on the caller's stream.
 // Precision (checked against an fp64 restatement at T=4096): the state is fed
 // to MFMA as bf16, U stays fp32 (it initialises the V' accumulator), the state
 // increment K^T V'' uses V'' split into bf16 hi + lo.
@@ -102,16 +103,26 @@ __device__ __forceinline__ bf16x8 pack_hi(f32x4 a, f32x4 b) {
   }
   return r;
 }
-__device__ __forceinline__ void pack_hilo(f32x4 a, f32x4 b, bf16x8 &hi, bf16x8 &lo) {
+typedef __attribute__((ext_vector_type(2))) float f32x2;
+typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
+__device__ __forceinline__ uint32_t cvt2(float a, float b) {  // one v_cvt_pk_bf16_f32
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{a, b}), bf16x2));
+}
+// x as bf16 hi + lo, converted in pairs (hi's values are its bits moved up)
+__device__ __forceinline__ void split4(f32x4 x, u32x2 &hi, u32x2 &lo) {
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const __bf16 ha = static_cast<__bf16>(a[i]);
-    const __bf16 hb = static_cast<__bf16>(b[i]);
-    hi[i] = ha;
-    hi[4 + i] = hb;
-    lo[i] = static_cast<__bf16>(a[i] - static_cast<float>(ha));
-    lo[4 + i] = static_cast<__bf16>(b[i] - static_cast<float>(hb));
+  for (int i = 0; i < 2; ++i) {
+    const uint32_t h = cvt2(x[2 * i], x[2 * i + 1]);
+    hi[i] = h;
+    lo[i] = cvt2(x[2 * i] - __uint_as_float(h << 16), x[2 * i + 1] - __uint_as_float(h & 0xffff0000u));
   }
+}
+__device__ __forceinline__ void pack_hilo(f32x4 a, f32x4 b, bf16x8 &hi, bf16x8 &lo) {
+  u32x2 ha, la, hb, lb;
+  split4(a, ha, la);
+  split4(b, hb, lb);
+  hi = as_bf16x8(u32x4{ha.x, ha.y, hb.x, hb.y});
+  lo = as_bf16x8(u32x4{la.x, la.y, lb.x, lb.y});
 }
 
 struct ChunkArgs {
@@ -132,24 +143,21 @@ struct ChunkArgs {
   float scale;
   int l2norm;
   int max_chunks;
-  int seg_begin, seg_end;  // global chunk range of this launch (workspace holds SEG chunks)
+  // This launch's segment (the workspace holds its chunks).  win == 0: the
+  // global chunks [seg_begin, seg_end), sequence after sequence; otherwise
+  // chunks [seg_begin, seg_begin + win) of every sequence, sequence n's in
+  // the slots from n * win.
+  int seg_begin, seg_end, win;
   // workspace
-  int32_t *chunk_start;  // [n_seqs + 2]: chunk starts, then the empty-sequence count
+  int32_t *chunk_start;  // [n_seqs + 1]: first global chunk of each sequence, and the total
   u32x4 *vh;             // [SEG][Hv][NB_VH][64]   -W, A, scalars
   float *Ut;             // [SEG][Hv][8 x 4 blocks][64][4]  U, fp32
   float *carry;          // [n_seqs][Hv][128][128] state between segments
-  int64_t *seqrec;       // [n_seqs][SEQREC]: per-sequence record for the persistent scan
   // [SEG][Hv / 2]: the chunk's q and k rows of v-head 2i + 1 equal those of 2i
   // (q and k given per v-head, Hk == Hv: the caller repeated them); null
   // unless the prep checks and the scan uses it
   int32_t *dup;
 };
-
-// Per-sequence record written by chunk_table_kernel for the persistent scan:
-// token start, state rows in / out (-1: none), end chunk, length, and the
-// next non-empty sequence (n_seqs: none).
-constexpr int SEQREC = 6;
-enum { SR_S0 = 0, SR_IN, SR_OUT, SR_CE, SR_LEN, SR_NXT };
 
 __device__ __forceinline__ void seq_bounds(const ChunkArgs &a, int n, int64_t *s0, int *len) {
   seq_range(a.cu, n, a.T, a.total, s0, len);
@@ -173,25 +181,16 @@ __device__ __forceinline__ void xcd_group_order(int bid, int per, int *g, int *m
 }
 
 // ------------------------------------------------------------------ chunk table
-// chunk_start[0 .. n_seqs]: first global chunk of each sequence (and the
-// total); chunk_start[n_seqs + 1]: the number of empty sequences.
+// chunk_start[0 .. n_seqs]: first global chunk of each sequence, and the total.
 __global__ __launch_bounds__(256) void chunk_table_kernel(ChunkArgs a) {
   __shared__ int32_t part[256];
-  __shared__ int32_t empties;
   int32_t carry = 0;
-  if (threadIdx.x == 0) {
-    a.chunk_start[0] = 0;
-    empties = 0;
-  }
-  __syncthreads();
+  if (threadIdx.x == 0) a.chunk_start[0] = 0;
   for (int base = 0; base < a.n_seqs; base += 256) {
     const int n = base + threadIdx.x;
     int64_t s0;
     int len = 0;
-    if (n < a.n_seqs) {
-      seq_bounds(a, n, &s0, &len);
-      if (len == 0) atomicAdd(&empties, 1);
-    }
+    if (n < a.n_seqs) seq_bounds(a, n, &s0, &len);
     part[threadIdx.x] = (len + CK - 1) / CK;
     __syncthreads();
     for (int off = 1; off < 256; off <<= 1) {  // inclusive scan
@@ -203,24 +202,6 @@ __global__ __launch_bounds__(256) void chunk_table_kernel(ChunkArgs a) {
     if (n < a.n_seqs) a.chunk_start[n + 1] = carry + part[threadIdx.x];
     carry += part[255];
     __syncthreads();
-  }
-  if (threadIdx.x == 0) a.chunk_start[a.n_seqs + 1] = empties;
-  __syncthreads();  // chunk_start complete (workgroup-visible)
-  for (int n = threadIdx.x; n < a.n_seqs; n += 256) {
-    int64_t s0;
-    int len;
-    seq_bounds(a, n, &s0, &len);
-    int k = n + 1;
-    while (k < a.n_seqs && a.chunk_start[k] == a.chunk_start[k + 1]) ++k;  // skip empty sequences
-    int64_t *r = a.seqrec + static_cast<int64_t>(n) * SEQREC;
-    r[SR_S0] = s0;
-    const int64_t rin = a.h0 ? pool_row(a.h0_idx, n, a.h0_rows) : -1;
-    const int64_t rout = a.hT ? pool_row(a.hT_idx, n, a.hT_rows) : -1;
-    r[SR_IN] = rin >= 0 && repeats_earlier_thread(a.h0_idx, n) ? -1 : rin;  // repeated slot ids: no row
-    r[SR_OUT] = rout >= 0 && repeats_earlier_thread(a.hT_idx, n) ? -1 : rout;
-    r[SR_CE] = a.chunk_start[n + 1];
-    r[SR_LEN] = len;
-    r[SR_NXT] = k;
   }
 }
 
@@ -358,22 +339,29 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void c
     h = (g % hg) * grp + m;
     jl = g / hg;
   }
-  const int j = a.seg_begin + jl;  // global chunk index
-  if (j >= a.seg_end || j >= chunk_start_at(a, a.n_seqs)) return;
-  int lo = 0, hi = a.n_seqs;  // sequence owning chunk j: last n with chunk_start[n] <= j
-  if (!a.cu) {
-    lo = j / ((a.T + CK - 1) / CK);
+  int n, c;  // the slot's sequence, and the chunk within it
+  if (a.win) {
+    n = jl / a.win;
+    c = a.seg_begin + jl % a.win;
+    if (n >= a.n_seqs) return;
   } else {
-    while (hi - lo > 1) {
-      const int mid = (lo + hi) >> 1;
-      if (a.chunk_start[mid] <= j) lo = mid; else hi = mid;
+    const int j = a.seg_begin + jl;  // global chunk index
+    if (j >= a.seg_end || j >= chunk_start_at(a, a.n_seqs)) return;
+    int lo = 0, hi = a.n_seqs;  // sequence owning chunk j: last n with chunk_start[n] <= j
+    if (!a.cu) {
+      lo = j / ((a.T + CK - 1) / CK);
+    } else {
+      while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (a.chunk_start[mid] <= j) lo = mid; else hi = mid;
+      }
     }
+    n = lo;
+    c = j - chunk_start_at(a, n);
   }
-  const int n = lo;
   int64_t s0;
   int slen;
   seq_bounds(a, n, &s0, &slen);
-  const int c = j - chunk_start_at(a, n);
   const int64_t t0 = s0 + static_cast<int64_t>(c) * CK;
   const int len = min(CK, slen - c * CK);
   if (len <= 0) {
@@ -664,7 +652,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void c
 // ------------------------------------------------------------------ phase B
 
 // sched_group_barrier masks
-constexpr int SG_MFMA = 0x8, SG_DS_RD = 0x100;
+constexpr int SG_VALU = 0x2, SG_MFMA = 0x8, SG_DS_RD = 0x100;
 #define GDN_SCHED_FENCE() __builtin_amdgcn_sched_barrier(0)
 #define GDN_GROUP(mask, n) __builtin_amdgcn_sched_group_barrier(mask, n, 0)
 
@@ -704,8 +692,7 @@ constexpr int RS_VH_COPIES = NB_VH - 2;
 constexpr int RS_LOADER0 = RS_VH_COPIES + 4;
 constexpr int RS_LOADER1 = 32;
 constexpr int SCAN_WAVES = 6;
-constexpr int SCAN_COLS = 16;  // state columns per workgroup
-constexpr int SCAN_PERSIST_BLOCKS = 256;  // one scan workgroup per CU (MI355X: 256 CUs)
+constexpr int SCAN_COLS = 16;  // state columns per workgroup of chunk_scan_kernel
 
 struct RowOps {     // one chunk's operands of one compute wave
   u32x4 w[4];       // -W rows 16q.., k-steps 0..3
@@ -715,59 +702,49 @@ struct RowOps {     // one chunk's operands of one compute wave
   f32x4 u, sk;      // U rows 16q + 4g + e of this lane's column; their V'' scales
   float sq, eL;     // output scale of position 16q + (lane % 16); e^{gamma_63}
 };
-// Token ranges of global chunks visited in increasing order (a scan
-// loader's walk): one search for the first chunk's sequence, then the next
-// sequence is entered when a chunk crosses the current one's end, with that
-// sequence's table entries read one crossing earlier.  Uniform; the chunk
-// table and cu_seqlens are read as scalar loads.
-struct ChunkWalk {
-  int n, cs, next_cs, slen;
-  int64_t s0;
-  int p_cs, p_slen;  // the next sequence's end chunk and length, read one crossing ahead
-  int64_t p_s0;
-  __device__ void prefetch(const ChunkArgs &a) {
-    const int m = min(n + 1, a.n_seqs - 1);
-    p_cs = chunk_start_at(a, m + 1);
-    seq_bounds(a, m, &p_s0, &p_slen);
-  }
-  __device__ void start(const ChunkArgs &a, int j) {
-    int lo = 0, hi = a.n_seqs;  // last n with chunk_start[n] <= j
-    if (!a.cu) {
-      lo = j / ((a.T + CK - 1) / CK);
-    } else {
-      while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
-        if (a.chunk_start[mid] <= j) lo = mid; else hi = mid;
-      }
-    }
-    n = lo;
-    cs = chunk_start_at(a, lo);
-    next_cs = chunk_start_at(a, lo + 1);
-    seq_bounds(a, lo, &s0, &slen);
-    prefetch(a);
-  }
-  // chunk j's first token and length (j at or after the previous call's)
-  __device__ void at(const ChunkArgs &a, int j, int64_t *t0, int *len) {
-    while (j >= next_cs && n + 1 < a.n_seqs) {  // (empty sequences have no chunks: cs == next_cs)
-      ++n;
-      cs = next_cs;
-      next_cs = p_cs;
-      s0 = p_s0;
-      slen = p_slen;
-      prefetch(a);
-    }
-    const int c = j - cs;
-    *t0 = s0 + static_cast<int64_t>(c) * CK;
-    *len = min(CK, slen - c * CK);
-  }
+// The chunks of one sequence that a scan workgroup walks in this launch.
+struct ScanRange {
+  int nch;      // chunks (0: none in this segment, or an empty sequence)
+  int c0;       // workspace slot of the first
+  int cs, ce;   // the sequence's chunks: within the sequence if win, else global
+  int lo, hi;   // of which this launch walks [lo, hi)
+  int64_t t0;   // first token of chunk lo
+  int rows;     // tokens from there to the sequence's end
 };
+__device__ __forceinline__ ScanRange scan_range(const ChunkArgs &a, int n) {
+  int64_t s0;
+  int slen;
+  seq_bounds(a, n, &s0, &slen);
+  s0 = uniform64(s0);
+  slen = __builtin_amdgcn_readfirstlane(slen);
+  ScanRange r;
+  if (a.win) {
+    r.cs = 0;
+    r.ce = (slen + CK - 1) / CK;
+    r.lo = min(a.seg_begin, r.ce);
+    r.hi = min(a.seg_begin + a.win, r.ce);
+    r.c0 = n * a.win;
+  } else {
+    r.cs = __builtin_amdgcn_readfirstlane(chunk_start_at(a, n));
+    r.ce = __builtin_amdgcn_readfirstlane(max(r.cs, min(chunk_start_at(a, n + 1), a.max_chunks)));
+    r.lo = max(r.cs, a.seg_begin);
+    r.hi = min(r.ce, a.seg_end);
+    r.c0 = r.lo - a.seg_begin;
+  }
+  r.nch = max(0, r.hi - r.lo);
+  r.t0 = s0 + static_cast<int64_t>(r.lo - r.cs) * CK;
+  r.rows = slen - (r.lo - r.cs) * CK;
+  return r;
+}
 struct RowSrc {     // one chunk's sources: its workspace regions (v-head operands, U) and raw k, q rows
   __amdgpu_buffer_rsrc_t vh, ut, k, q;
 };
-// ch: the (chunk, v-head) index within the workspace; the chunk's tokens
-// [t0, t0 + len).  Rows past the chunk's end read as zero (their offsets are
-// range checked).
-__device__ __forceinline__ RowSrc row_src(const ChunkArgs &a, size_t ch, int64_t t0, int len, int hk) {
+// The sources of chunk c of the range.  Rows past the sequence's end read as
+// zero (their offsets are range checked).
+__device__ __forceinline__ RowSrc row_src(const ChunkArgs &a, const ScanRange &sr, int c, int h, int hk) {
+  const size_t ch = static_cast<size_t>(sr.c0 + c) * a.Hv + h;
+  const int64_t t0 = sr.t0 + static_cast<int64_t>(c) * CK;
+  const int len = min(CK, sr.rows - c * CK);
   const int64_t kb = (len - 1) * a.ks * 2 + DK * 2, qb = (len - 1) * a.qs * 2 + DK * 2;
   return RowSrc{__builtin_amdgcn_make_buffer_rsrc(a.vh + ch * (NB_VH * 64), 0, NB_VH * 1024, BUF_DWORD3),
                 __builtin_amdgcn_make_buffer_rsrc(a.Ut + ch * (DV * CK), 0, DV * CK * 4, BUF_DWORD3),
@@ -863,10 +840,10 @@ __device__ __forceinline__ u32x2 pack4(f32x4 x) {
 // registers of an A operand are those of the transposed B operand, so sb,
 // the V' exchange and the Q and A blocks serve unchanged, and lane (g, r)
 // ends with O[16q + r][4g .. 4g + 3], one 8-byte store.
-template <bool TWO_A, class StoreOut, class AtState>
+template <bool TWO_A, class StoreOut>
 __device__ __forceinline__ void scan_rows_chunk(const RowOps &op, RowOps &nx, const u32x4 *nst, bf16x8 (&sb)[4],
                                                 f32x4 (&S)[2], u32x2 (*xv)[2][64][2], u32x4 (*xs)[64], int q,
-                                                int lane, const StoreOut &store_out, const AtState &at_state) {
+                                                int lane, const StoreOut &store_out) {
   // ---- R1
   f32x4 vp = op.u;
 #pragma unroll
@@ -919,7 +896,6 @@ __device__ __forceinline__ void scan_rows_chunk(const RowOps &op, RowOps &nx, co
     GDN_GROUP(SG_DS_RD, 2);
   }
   GDN_SCHED_FENCE();
-  at_state(S);  // (persistent scan: a sequence that ends here hands over to the next one's initial state)
   xs[q][lane] = __builtin_bit_cast(u32x4, pack_hi(S[0], S[1]));
   lds_barrier();
 
@@ -942,19 +918,12 @@ constexpr int vmcnt_only(int n) { return 0x0F70 | (n & 15) | ((n >> 4) << 14); }
 // barriers carry no fence (a release fence would wait for every copy in
 // flight, including those for the chunk after next).
 template <int LD>
-__device__ __forceinline__ void scan_rows_loader(u32x4 (*stage)[RS_BLOCKS * 64], int nch, int ct, int lane,
-                                                 const ChunkArgs &a, int c0, int h, int hk) {
+__device__ __forceinline__ void scan_rows_loader(u32x4 (*stage)[RS_BLOCKS * 64], int ct, int lane, const ChunkArgs &a,
+                                                 const ScanRange &sr, int h, int hk) {
   constexpr int N = LD == 0 ? RS_LOADER0 : RS_LOADER1;  // copies per chunk
   constexpr int H = N / 2;                               // of which before barrier 1
-  ChunkWalk walk;
-  walk.start(a, a.seg_begin + c0);
-  auto src_of = [&](int c) {  // (called with increasing c)
-    const size_t j = static_cast<size_t>(c0 + c);
-    int64_t t0;
-    int len;
-    walk.at(a, a.seg_begin + c0 + c, &t0, &len);
-    return row_src(a, j * a.Hv + h, t0, len, hk);
-  };
+  const int nch = sr.nch;
+  auto src_of = [&](int c) { return row_src(a, sr, c, h, hk); };
   stage_copy<LD>(stage[0], src_of(0), a, ct, 0, N, lane);
   if (nch > 1) {
     stage_copy<LD>(stage[1], src_of(1), a, ct, 0, N, lane);
@@ -1005,18 +974,11 @@ __global__ __launch_bounds__(64 * SCAN_WAVES) void chunk_scan_kernel(ChunkArgs a
   int hk = h / ratio;
   const int col = 16 * ct + (lane & 15);
 
-  int64_t s0;
-  int slen;
-  seq_bounds(a, n, &s0, &slen);
-  s0 = uniform64(s0);
-  slen = __builtin_amdgcn_readfirstlane(slen);
-  const int cs = __builtin_amdgcn_readfirstlane(chunk_start_at(a, n));
-  const int ce = __builtin_amdgcn_readfirstlane(max(cs, min(chunk_start_at(a, n + 1), a.max_chunks)));
-  const int lo = max(cs, a.seg_begin), hi = min(ce, a.seg_end);
+  const ScanRange sr = scan_range(a, n);
   const int64_t in_row = a.h0 ? uniform64(pool_row_first(a.h0_idx, n, a.h0_rows)) : -1;
   const int64_t out_row = a.hT ? uniform64(pool_row_first(a.hT_idx, n, a.hT_rows)) : -1;
   const int64_t kv = static_cast<int64_t>(DK) * DV;
-  if (cs == ce) {  // empty sequence: the final state is the initial one (handled once)
+  if (sr.cs == sr.ce) {  // empty sequence: the final state is the initial one (handled once)
     if (wave < 4 && a.seg_begin == 0 && out_row >= 0) {
       float *dst = a.hT + (out_row * a.Hv + h) * kv + col;
 #pragma unroll
@@ -1029,29 +991,27 @@ __global__ __launch_bounds__(64 * SCAN_WAVES) void chunk_scan_kernel(ChunkArgs a
     }
     return;
   }
-  if (lo >= hi) return;  // no chunk of this sequence in this segment
-  const int nch = hi - lo;
-  const int c0 = lo - a.seg_begin;                             // first chunk, workspace-local
-  const int64_t seq_off = static_cast<int64_t>(lo - cs) * CK;  // its first token within the sequence
+  const int nch = sr.nch;
+  if (nch == 0) return;  // no chunk of this sequence in this segment
   if (a.dup && (h & 1)) {  // every chunk of the range repeats the even partner's q / k rows: read that copy
     bool all = true;
     for (int i0 = 0; i0 < nch; i0 += 64) {
       const int i = i0 + lane;
-      all = all && __all(i >= nch || a.dup[(c0 + i) * (a.Hv / 2) + h / 2] != 0);
+      all = all && __all(i >= nch || a.dup[(sr.c0 + i) * (a.Hv / 2) + h / 2] != 0);
     }
     if (all) hk = h - 1;
   }
   if (wave >= 4) {
     if (wave == 4)
-      scan_rows_loader<0>(stage, nch, ct, lane, a, c0, h, hk);
+      scan_rows_loader<0>(stage, ct, lane, a, sr, h, hk);
     else
-      scan_rows_loader<1>(stage, nch, ct, lane, a, c0, h, hk);
+      scan_rows_loader<1>(stage, ct, lane, a, sr, h, hk);
     return;
   }
   float *carry = a.carry + (static_cast<int64_t>(n) * a.Hv + h) * kv + col;
 
   f32x4 S[2];  // tiles 2q, 2q + 1: state rows key_dim(2q + t, g, e) of this lane's column
-  const float *src = lo == cs ? (in_row >= 0 ? a.h0 + (in_row * a.Hv + h) * kv + col : nullptr) : carry;
+  const float *src = sr.lo == sr.cs ? (in_row >= 0 ? a.h0 + (in_row * a.Hv + h) * kv + col : nullptr) : carry;
   if (src) {
 #pragma unroll
     for (int t = 0; t < 2; ++t)
@@ -1069,9 +1029,8 @@ __global__ __launch_bounds__(64 * SCAN_WAVES) void chunk_scan_kernel(ChunkArgs a
   const int64_t ostep = static_cast<int64_t>(a.Hv) * DV;  // elements per token
   const int voff = static_cast<int>(((16 * q + (lane & 15)) * ostep + h * DV + 16 * ct + 4 * g4) * sizeof(OT));
   auto store_out = [&](const f32x4 &o, int c) {  // chunk c of this launch: rows [0, min(64, rest of sequence))
-    const int64_t toff = seq_off + static_cast<int64_t>(c) * CK;
-    const int rows = static_cast<int>(min<int64_t>(CK, slen - toff));
-    OT *base = static_cast<OT *>(a.o) + (s0 + toff) * ostep;
+    const int rows = min(CK, sr.rows - c * CK);
+    OT *base = static_cast<OT *>(a.o) + (sr.t0 + static_cast<int64_t>(c) * CK) * ostep;
     const auto r = __builtin_amdgcn_make_buffer_rsrc(base, 0, static_cast<int>(rows * ostep * sizeof(OT)), BUF_DWORD3);
     if constexpr (BF16_OUT)
       __builtin_amdgcn_raw_buffer_store_b64(pack4(o), r, voff, 0, 0);
@@ -1083,11 +1042,10 @@ __global__ __launch_bounds__(64 * SCAN_WAVES) void chunk_scan_kernel(ChunkArgs a
     // (after the last chunk the "next" reads take the idle buffer's stale contents, unused)
     const u32x4 *nst = stage[(c + 1) & 1];
     auto out = [&](const f32x4 &o) { store_out(o, c); };
-    auto keep = [](f32x4 (&)[2]) {};
     if (q >= 2)
-      scan_rows_chunk<true>(op, nx, nst, sb, S, xv, xs, q, lane, out, keep);
+      scan_rows_chunk<true>(op, nx, nst, sb, S, xv, xs, q, lane, out);
     else
-      scan_rows_chunk<false>(op, nx, nst, sb, S, xv, xs, q, lane, out, keep);
+      scan_rows_chunk<false>(op, nx, nst, sb, S, xv, xs, q, lane, out);
   };
 
   RowOps op0, op1;
@@ -1108,7 +1066,7 @@ __global__ __launch_bounds__(64 * SCAN_WAVES) void chunk_scan_kernel(ChunkArgs a
     chunk(op1, op0, c + 1);
   }
 
-  float *dst = hi == ce ? (out_row >= 0 ? a.hT + (out_row * a.Hv + h) * kv + col : nullptr) : carry;
+  float *dst = sr.hi == sr.ce ? (out_row >= 0 ? a.hT + (out_row * a.Hv + h) * kv + col : nullptr) : carry;
   if (dst) {
 #pragma unroll
     for (int t = 0; t < 2; ++t)
@@ -1117,189 +1075,314 @@ __global__ __launch_bounds__(64 * SCAN_WAVES) void chunk_scan_kernel(ChunkArgs a
   }
 }
 
-// Persistent scan for several sequences (varlen or a dense batch): one
-// workgroup per (v-head, 16 state columns) walks every chunk of the segment
-// in order, sequence after sequence, instead of one workgroup per
-// (sequence, v-head, columns) paying its start and end for a few chunks each.
-// The loader waves stream the segment's chunks as for one sequence; the
-// compute waves track the sequence of each chunk, and where one ends (after
-// its last state update, before the state exchange) they store its final
-// state and continue from the next one's initial state, loaded into
-// registers a sequence ahead.  Used when (v-heads x column tiles) alone fill
-// the CUs.
-template <bool BF16_OUT>
-__global__ __launch_bounds__(64 * SCAN_WAVES) void chunk_scan_persist_kernel(ChunkArgs a) {
-  __shared__ u32x4 stage[2][RS_BLOCKS * 64];  // 122 KiB
-  __shared__ u32x4 xs[4][64];
-  __shared__ u32x2 xv[3][2][64][2];
+// ------------------------------------------------------------ column scan
+// The scan of several sequences: one workgroup of NW compute waves and two
+// loader waves per (sequence, v-head, 16 NW state columns), so that every
+// sequence's chain runs at once (one workgroup per (v-head, 16 columns) walking
+// the sequences one after the other took B = 2 / 3 / 4 x T = 1038 59.3 / 85.7 /
+// 130.1 us, this 48.0 / 64.8 / 92.4; B = 4 x T = 4096 413 -> 305).  Each compute wave owns 16 state columns for
+// the whole sequence (all 128 rows in eight accumulator tiles), so it needs
+// no other wave's values: the state is the B operand of V' and the A operand
+// of O^T straight from the accumulators (pi order), V'' that of the update.
+// LDS holds only the operands, double-buffered and shared by the NW waves
+// (-W, A, scalars, the raw k and q rows and the waves' U tiles).  Step c:
+//   R1  V' = U - W S              | k rows and scalars of c read | barrier A
+//   R2  S <- e^{gamma_63} S + K^T V''      | q rows of c read    | barrier B
+//   R3  O^T = (S^T Q^T) diag(sq) + V'^T A^T | -W, U of c + 1, A of c read
+// (each region's LDS reads run behind its products).  A step takes 2,530 cycles
+// with 2 waves and 3,240 with 4 (1.17 / 1.48 us, from s_memtime stamps): R1 780 /
+// 1,040, bound by its LDS reads (32 transposing reads per wave on top of its
+// neighbours'), R2 840 / 990, about 100 vector instructions and 32 MFMAs, R3
+// 730 / 900.  The loaders refill what
+// a barrier releases and wait for what the next regions read, 1.5 steps after
+// its request:
+//   after A(c) they request -W, U, scalars and k of c + 2 and A of c + 1, due before B(c + 1);
+//   after B(c) q of c + 2, due before A(c + 2).
+constexpr int CS_U = RS_U;  // stage blocks: the v-head region, K and Q rows, then the U tiles
+constexpr int cs_blocks(int nw) { return CS_U + 4 * nw; }
+constexpr int CS_A0 = NB_W, CS_SC = NB_W + 6;  // loader 0's copies: -W [0, 16), A [16, 22), scalars
+static_assert(RS_VH_COPIES == CS_SC + 1, "loader 0's order");
+
+// U blocks u0 .. u0 + n of one chunk into st.
+__device__ __forceinline__ void stage_copy_u(u32x4 *st, const RowSrc &r, int n, int u0, int lane) {
+  for (int i = 0; i < n; ++i)
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r.ut, st + i * 64, 16, lane * 16, (u0 + i) * 1024, 0, 0);
+}
+
+template <int LD, int NW>
+__device__ __forceinline__ void scan_cols_loader(u32x4 *stage, int tile, int lane, const ChunkArgs &a,
+                                                 const ScanRange &sr, int h, int hk) {
+  const int nch = sr.nch;
+  auto src_of = [&](int c) { return row_src(a, sr, c, h, hk); };
+  auto buf = [&](int c) { return stage + (c & 1) * (cs_blocks(NW) * 64); };
+  RowSrc r1 = src_of(0), r2 = r1;  // of chunks c + 1 and c + 2
+  if constexpr (LD == 0) {
+    constexpr int G = NB_W + 4 * NW + 1;
+    auto wus = [&](int c, const RowSrc &r) {
+      stage_copy<0>(buf(c), r, a, 0, 0, NB_W, lane);
+      stage_copy_u(buf(c) + CS_U * 64, r, 4 * NW, 4 * NW * tile, lane);
+      stage_copy<0>(buf(c), r, a, 0, CS_SC, CS_SC + 1, lane);
+    };
+    auto ablk = [&](int c, const RowSrc &r) { stage_copy<0>(buf(c), r, a, 0, CS_A0, CS_SC, lane); };
+    wus(0, r1);
+    if (nch > 1) {
+      r2 = src_of(1);
+      wus(1, r2);
+    }
+    ablk(0, r1);
+    if (nch > 1) __builtin_amdgcn_s_waitcnt(vmcnt_only(G + 6));
+    else __builtin_amdgcn_s_waitcnt(vmcnt_only(6));
+    __builtin_amdgcn_s_barrier();  // B before chunk 0
+    for (int c = 0; c < nch; ++c) {
+      __builtin_amdgcn_s_barrier();  // A
+      r1 = r2;
+      if (c + 2 < nch) {
+        r2 = src_of(c + 2);
+        wus(c + 2, r2);
+        ablk(c + 1, r1);
+        __builtin_amdgcn_s_waitcnt(vmcnt_only(G + 6));
+      } else if (c + 1 < nch) {
+        ablk(c + 1, r1);
+        __builtin_amdgcn_s_waitcnt(vmcnt_only(6));
+      } else {
+        __builtin_amdgcn_s_waitcnt(vmcnt_only(0));
+      }
+      __builtin_amdgcn_s_barrier();  // B
+    }
+  } else {
+    auto krows = [&](int c, const RowSrc &r) { stage_copy<1>(buf(c), r, a, 0, 0, 16, lane); };
+    auto qrows = [&](int c, const RowSrc &r) { stage_copy<1>(buf(c), r, a, 0, 16, 32, lane); };
+    krows(0, r1);
+    qrows(0, r1);
+    if (nch > 1) {
+      r2 = src_of(1);
+      krows(1, r2);
+      __builtin_amdgcn_s_waitcnt(vmcnt_only(32));
+    } else {
+      __builtin_amdgcn_s_waitcnt(vmcnt_only(16));
+    }
+    __builtin_amdgcn_s_barrier();  // B before chunk 0
+    if (nch > 1) qrows(1, r2);
+    for (int c = 0; c < nch; ++c) {
+      if (c + 1 < nch) __builtin_amdgcn_s_waitcnt(vmcnt_only(32));
+      else __builtin_amdgcn_s_waitcnt(vmcnt_only(0));
+      __builtin_amdgcn_s_barrier();  // A
+      const bool more = c + 2 < nch;
+      if (more) {
+        r2 = src_of(c + 2);
+        krows(c + 2, r2);
+        __builtin_amdgcn_s_waitcnt(vmcnt_only(32));
+      } else {
+        __builtin_amdgcn_s_waitcnt(vmcnt_only(16));
+      }
+      __builtin_amdgcn_s_barrier();  // B
+      if (more) qrows(c + 2, r2);
+    }
+  }
+}
+
+template <int NW, bool BF16_OUT>
+__global__ __launch_bounds__(64 * (NW + 2)) __attribute__((amdgpu_waves_per_eu(1, 2))) void chunk_scan_cols_kernel(ChunkArgs a) {
+  constexpr int TILES = DV / (16 * NW);  // workgroups per (sequence, v-head)
+  __shared__ u32x4 stage[2][cs_blocks(NW) * 64];  // 130 or 146 KiB
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int q = wave & 3;
-  const int g4 = lane >> 4;
+  const int g4 = lane >> 4, r16 = lane & 15;
   const int ratio = a.Hv / a.Hk;
-  int ct = blockIdx.x / a.Hv;
-  int h = blockIdx.x % a.Hv;
-  if (a.Hk % 8 == 0) {  // the column tiles and v-heads of one k-head on one XCD
+  const int grp = a.dup ? 2 : ratio, hg = a.Hv / grp;  // v-heads reading the same q / k rows: on one XCD
+  int tile = blockIdx.x % TILES, rest = blockIdx.x / TILES;
+  if ((a.n_seqs * hg) % 8 == 0) {
     int g, m;
-    xcd_group_order(blockIdx.x, ratio * (DV / SCAN_COLS), &g, &m);
-    ct = m % (DV / SCAN_COLS);
-    h = g * ratio + m / (DV / SCAN_COLS);
+    xcd_group_order(blockIdx.x, grp * TILES, &g, &m);
+    tile = m % TILES;
+    rest = (g / hg) * a.Hv + (g % hg) * grp + m / TILES;
   }
-  const int hk = h / ratio;
-  const int col = 16 * ct + (lane & 15);
-  const int64_t kv = static_cast<int64_t>(DK) * DV;
-  auto state_at = [&](float *base, int64_t row) { return base + (row * a.Hv + h) * kv + col; };
-  auto load_state = [&](const float *src, f32x4 (&S)[2]) {
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) S[t][e] = src ? src[key_dim(2 * q + t, g4, e) * DV] : 0.f;
-  };
-  auto store_state = [&](float *dst, const f32x4 (&S)[2]) {
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) dst[key_dim(2 * q + t, g4, e) * DV] = S[t][e];
-  };
-  auto init_src = [&](int64_t row) -> const float * {
-    return row >= 0 ? state_at(const_cast<float *>(a.h0), row) : nullptr;
-  };
-  // sequence records (chunk_table_kernel, read-only here): uniform, so read
-  // through the constant address space as scalar loads into SGPRs
-  typedef const __attribute__((address_space(4))) int64_t crec_t;
-  crec_t *recp = (crec_t *)(a.seqrec);
-  struct Rec {
-    int64_t s0, in, out;
-    int ce, len, nxt;
-  };
-  const bool arith = !a.cu && !a.h0_idx && !a.hT_idx;  // a dense batch without slot ids: no table
-  auto rec_get = [&](int m) -> Rec {
-    if (arith) {
-      const int cpb = (a.T + CK - 1) / CK;
-      return Rec{static_cast<int64_t>(m) * a.T, a.h0 ? pool_row(nullptr, m, a.h0_rows) : -1,
-                 a.hT ? pool_row(nullptr, m, a.hT_rows) : -1, (m + 1) * cpb, a.T, m + 1};
-    }
-    crec_t *r = recp + static_cast<int64_t>(m) * SEQREC;
-    return Rec{r[SR_S0], r[SR_IN], r[SR_OUT], static_cast<int>(r[SR_CE]), static_cast<int>(r[SR_LEN]),
-               static_cast<int>(r[SR_NXT])};
-  };
+  const int n = rest / a.Hv, h = rest % a.Hv;
+  int hk = h / ratio;
+  const int ct = NW * tile + wave;  // a compute wave's column tile
+  const int col = 16 * ct + r16;
 
-  const int lo = a.seg_begin, hi = min(a.seg_end, chunk_start_at(a, a.n_seqs));
-  const bool any_empty = a.cu ? a.chunk_start[a.n_seqs + 1] > 0 : a.T == 0;  // (counted by the table kernel)
-  if (wave < 4 && a.seg_begin == 0 && any_empty) {  // empty sequences pass their initial state through
-    for (int m = 0; m < a.n_seqs; ++m) {
-      if (chunk_start_at(a, m) != chunk_start_at(a, m + 1)) continue;
-      const Rec r = rec_get(m);
-      if (r.out < 0) continue;
-      f32x4 Sx[2];
-      load_state(init_src(r.in), Sx);
-      store_state(state_at(a.hT, r.out), Sx);
+  const ScanRange sr = scan_range(a, n);
+  const int64_t in_row = a.h0 ? uniform64(pool_row_first(a.h0_idx, n, a.h0_rows)) : -1;
+  const int64_t out_row = a.hT ? uniform64(pool_row_first(a.hT_idx, n, a.hT_rows)) : -1;
+  const int64_t kv = static_cast<int64_t>(DK) * DV;
+  const bool empty = sr.cs == sr.ce;
+  const int nch = sr.nch;
+  if (empty ? a.seg_begin != 0 || out_row < 0 : nch == 0) return;  // nothing to do in this segment
+  if (a.dup && (h & 1) && nch > 0) {  // every chunk of the range repeats the even partner's q / k rows: read that copy
+    bool all = true;
+    for (int i0 = 0; i0 < nch; i0 += 64) {
+      const int i = i0 + lane;
+      all = all && __all(i >= nch || a.dup[(sr.c0 + i) * (a.Hv / 2) + h / 2] != 0);
     }
+    if (all) hk = h - 1;
   }
-  if (lo >= hi) return;
-  const int nch = hi - lo;
-  if (wave >= 4) {
-    if (wave == 4)
-      scan_rows_loader<0>(stage, nch, ct, lane, a, 0, h, hk);
+  if (wave >= NW) {
+    if (nch == 0) return;
+    if (wave == NW)
+      scan_cols_loader<0, NW>(stage[0], tile, lane, a, sr, h, hk);
     else
-      scan_rows_loader<1>(stage, nch, ct, lane, a, 0, h, hk);
+      scan_cols_loader<1, NW>(stage[0], tile, lane, a, sr, h, hk);
     return;
   }
 
-  // the sequence of chunk lo: the last one starting at or before it (non-empty)
-  int n;
+  float *carry = a.carry + (static_cast<int64_t>(n) * a.Hv + h) * kv + col;
+  f32x4 S[8];  // tile t: state rows key_dim(t, g, e) of this lane's column
   {
-    int l = 0, r = a.n_seqs;
-    while (r - l > 1) {
-      const int mid = (l + r) >> 1;
-      if (chunk_start_at(a, mid) <= lo) l = mid; else r = mid;
-    }
-    n = __builtin_amdgcn_readfirstlane(l);
-  }
-  // Current sequence n, the next one nn (its record and initial state Sn in
-  // registers) and the one after, nnn (its record requested): at a sequence
-  // end what the next sequence needs is already loaded.
-  float *carry = a.carry;
-  f32x4 S[2], Sn[2];
-  const Rec rc = rec_get(n);
-  int cs = __builtin_amdgcn_readfirstlane(chunk_start_at(a, n));
-  int ce = rc.ce, slen = rc.len;
-  int64_t s0 = rc.s0, orow = rc.out;
-  load_state(lo == cs ? init_src(rc.in) : state_at(carry, n), S);
-  int nn = ce < hi ? rc.nxt : a.n_seqs;
-  int nnn = a.n_seqs;
-  Rec rn{0, -1, -1, 0, 0, 0}, r3{0, -1, -1, 0, 0, 0};
-  auto take_next = [&]() {  // rn = nn's record: its initial state, and nnn's record
-    load_state(init_src(rn.in), Sn);
-    nnn = rn.ce < hi ? rn.nxt : a.n_seqs;
-    if (nnn < a.n_seqs) r3 = rec_get(nnn);
-  };
-  if (nn < a.n_seqs) {
-    rn = rec_get(nn);
-    take_next();
-  }
-
-  typedef typename std::conditional<BF16_OUT, uint16_t, float>::type OT;
-  const int64_t ostep = static_cast<int64_t>(a.Hv) * DV;
-  const int voff = static_cast<int>(((16 * q + (lane & 15)) * ostep + h * DV + 16 * ct + 4 * g4) * sizeof(OT));
-  bf16x8 sb[4];
-  auto chunk = [&](const RowOps &op, RowOps &nx, int c) {
-    const u32x4 *nst = stage[(c + 1) & 1];
-    const int j = lo + c;  // global chunk, in sequence n
-    const int64_t toff = static_cast<int64_t>(j - cs) * CK;
-    const int rows = static_cast<int>(min<int64_t>(CK, slen - toff));
-    OT *base = static_cast<OT *>(a.o) + (s0 + toff) * ostep;
-    auto out = [base, rows, ostep, voff](const f32x4 &o) {
-      const auto r = __builtin_amdgcn_make_buffer_rsrc(base, 0, static_cast<int>(rows * ostep * sizeof(OT)), BUF_DWORD3);
-      if constexpr (BF16_OUT)
-        __builtin_amdgcn_raw_buffer_store_b64(pack4(o), r, voff, 0, 0);
-      else
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, o), r, voff, 0, 0);
-    };
-    auto at_state = [&](f32x4 (&St)[2]) {
-      if (j + 1 == ce && j + 1 < hi) {  // sequence n ends here, sequence nn starts with the next chunk
-        if (orow >= 0) store_state(state_at(a.hT, orow), St);
-        St[0] = Sn[0];
-        St[1] = Sn[1];
-        n = nn;
-        cs = ce;
-        ce = rn.ce;
-        s0 = rn.s0;
-        slen = rn.len;
-        orow = rn.out;
-        nn = nnn;
-        if (nn < a.n_seqs) {
-          rn = r3;
-          take_next();
-        }
-      }
-    };
-    if (q >= 2)
-      scan_rows_chunk<true>(op, nx, nst, sb, S, xv, xs, q, lane, out, at_state);
-    else
-      scan_rows_chunk<false>(op, nx, nst, sb, S, xv, xs, q, lane, out, at_state);
-  };
-
-  RowOps op0, op1;
-  xs[q][lane] = __builtin_bit_cast(u32x4, pack_hi(S[0], S[1]));
-  lds_barrier();  // state exchange; chunk 0 staged
+    const float *src = sr.lo == sr.cs ? (in_row >= 0 ? a.h0 + (in_row * a.Hv + h) * kv + col : nullptr) : carry;
 #pragma unroll
-  for (int s = 0; s < 4; ++s) sb[s] = __builtin_bit_cast(bf16x8, xs[s][lane]);
-  read_rows<0>(op0, stage[0], q, lane);
-  read_rows<1>(op0, stage[0], q, lane);
-  read_rows<2>(op0, stage[0], q, lane);
-  read_rows<3>(op0, stage[0], q, lane);
-  lds_barrier();  // chunk 0 read: its buffer may be refilled
-  for (int c = 0; c < nch; c += 2) {
-    chunk(op0, op1, c);
-    if (c + 1 >= nch) break;
-    chunk(op1, op0, c + 1);
+    for (int t = 0; t < 8; ++t)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) S[t][e] = src ? src[key_dim(t, g4, e) * DV] : 0.f;
   }
-  // the last sequence: finished here, or continued by the next segment
-  if (ce <= hi) {
-    if (orow >= 0) store_state(state_at(a.hT, orow), S);
-  } else {
-    store_state(state_at(carry, n), S);
+  typedef typename std::conditional<BF16_OUT, uint16_t, float>::type OT;
+  const int64_t ostep = static_cast<int64_t>(a.Hv) * DV;  // elements per token
+  const int voff = static_cast<int>((r16 * ostep + h * DV + 16 * ct + 4 * g4) * sizeof(OT));
+  // LDS byte offsets of this lane's operands, shared by both buffers: the
+  // fragments of the tiles and k-steps lie a constant apart (frag_kt and
+  // frag_row's addresses; only the segment's upper two bits need a register)
+  int koff[4], qoff[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    koff[i] = 2 * nsw(4 * g4 + (r16 >> 2), 32 * i + 8 * (r16 & 3));
+    qoff[i] = 2 * nsw(r16, 32 * i + 8 * g4);
+  }
+  u32x4 w[16];  // the next chunk's -W blocks
+  f32x4 u[4];   // and its U tiles of these columns
+  auto read_w = [&](const char *st) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) w[i] = *reinterpret_cast<const u32x4 *>(st + lane * 16 + (RS_VH + VH_W + i) * 1024);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) u[i] = *reinterpret_cast<const f32x4 *>(st + lane * 16 + wave * 4096 + (CS_U + i) * 1024);
+  };
+  const char *const buf0 = reinterpret_cast<const char *>(stage[0]), *const buf1 = reinterpret_cast<const char *>(stage[1]);
+  if (nch > 0) {
+    lds_barrier();  // B before chunk 0
+    read_w(buf0);
+  }
+  auto chunk = [&](const char *st, const char *nst, int c) {
+    const float *sc = reinterpret_cast<const float *>(st + (RS_VH + VH_SC) * 1024);
+    // ---- R1
+    bf16x8 kt[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {  // k-step i / 8, tile i % 8
+      const char *kp = st + koff[(i & 7) >> 1] + (RS_K * 1024 + (i >> 3) * 8192 + (i & 1) * 8);
+      const s16x4 k0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4 *)(const_cast<char *>(kp)));
+      const s16x4 k1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4 *)(const_cast<char *>(kp + 4096)));
+      kt[i] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(k0, k1, 0, 1, 2, 3, 4, 5, 6, 7));
+    }
+    const float eL = sc[2 * CK];
+    float sq[4];
+    f32x4 sk[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      sk[t] = *reinterpret_cast<const f32x4 *>(sc + CK + 16 * t + 4 * g4);
+      sq[t] = sc[16 * t + r16];
+    }
+    bf16x8 sb[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) sb[s] = pack_hi(S[2 * s], S[2 * s + 1]);
+    f32x4 vp[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) vp[t] = u[t];
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) vp[t] = mfma(as_bf16x8(w[4 * t + s]), sb[s], vp[t]);
+#pragma unroll
+    for (int t = 0; t < 8; ++t) S[t] = S[t] * eL;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      GDN_GROUP(SG_MFMA, 1);
+      GDN_GROUP(SG_DS_RD, 3);
+      GDN_GROUP(SG_VALU, 3);
+    }
+    GDN_SCHED_FENCE();
+    lds_barrier();  // A
+
+    // ---- R2
+    bf16x8 vb[2], vh[2], vl[2];
+    pack_hilo(vp[0] * sk[0], vp[1] * sk[1], vh[0], vl[0]);
+    GDN_SCHED_FENCE();
+#pragma unroll
+    for (int t = 0; t < 8; ++t) S[t] = mfma(kt[t], vh[0], S[t]);
+#pragma unroll
+    for (int t = 0; t < 8; ++t) S[t] = mfma(kt[t], vl[0], S[t]);
+    pack_hilo(vp[2] * sk[2], vp[3] * sk[3], vh[1], vl[1]);
+    vb[0] = pack_hi(vp[0], vp[1]);
+    vb[1] = pack_hi(vp[2], vp[3]);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      GDN_GROUP(SG_MFMA, 1);
+      GDN_GROUP(SG_VALU, 3);
+    }
+    GDN_SCHED_FENCE();
+    bf16x8 qf[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i)  // k-step i / 4, positions 16 (i % 4) + r
+      qf[i] = as_bf16x8(*reinterpret_cast<const u32x4 *>(st + qoff[i >> 2] + (RS_Q * 1024 + (i & 3) * 4096)));
+#pragma unroll
+    for (int t = 0; t < 8; ++t) S[t] = mfma(kt[8 + t], vh[1], S[t]);
+#pragma unroll
+    for (int t = 0; t < 8; ++t) S[t] = mfma(kt[8 + t], vl[1], S[t]);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      GDN_GROUP(SG_MFMA, 1);
+      GDN_GROUP(SG_DS_RD, 1);
+    }
+    GDN_SCHED_FENCE();
+    lds_barrier();  // B
+
+    // ---- R3
+    u32x4 ab[6];
+#pragma unroll
+    for (int i = 0; i < 6; ++i)
+      ab[i] = *reinterpret_cast<const u32x4 *>(st + lane * 16 + (RS_VH + VH_A + (i < 2 ? 2 * i : i + 2)) * 1024);
+    f32x4 o[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o[i] = mfma(sb[s], qf[4 * s + i], o[i]);
+    read_w(nst);  // (after the last chunk: stale contents, unused)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      GDN_GROUP(SG_MFMA, 1);
+      GDN_GROUP(SG_DS_RD, 2);
+    }
+    GDN_SCHED_FENCE();
+    const int rows = min(CK, sr.rows - c * CK);
+    const auto ro = __builtin_amdgcn_make_buffer_rsrc(
+        static_cast<OT *>(a.o) + (sr.t0 + static_cast<int64_t>(c) * CK) * ostep, 0,
+        static_cast<int>(rows * ostep * sizeof(OT)), BUF_DWORD3);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) o[i] = o[i] * sq[i];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) o[i] = mfma(vb[0], as_bf16x8(ab[i < 2 ? i : 2 * i - 2]), o[i]);
+#pragma unroll
+    for (int i = 2; i < 4; ++i) o[i] = mfma(vb[1], as_bf16x8(ab[2 * i - 1]), o[i]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int ioff = voff + static_cast<int>(16 * i * ostep * sizeof(OT));
+      if constexpr (BF16_OUT)
+        __builtin_amdgcn_raw_buffer_store_b64(pack4(o[i]), ro, ioff, 0, 0);
+      else
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, o[i]), ro, ioff, 0, 0);
+    }
+    GDN_SCHED_FENCE();
+  };
+  for (int c = 0; c < nch; c += 2) {  // (each buffer's LDS addresses stay in registers)
+    chunk(buf0, buf1, c);
+    if (c + 1 >= nch) break;
+    chunk(buf1, buf0, c + 1);
+  }
+  float *dst = empty || sr.hi == sr.ce ? (out_row >= 0 ? a.hT + (out_row * a.Hv + h) * kv + col : nullptr) : carry;
+  if (dst) {
+#pragma unroll
+    for (int t = 0; t < 8; ++t)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) dst[key_dim(t, g4, e) * DV] = S[t][e];
   }
 }
 
@@ -1879,6 +1962,12 @@ __global__ __launch_bounds__(64 * LOC_WAVES) void chunk_local_kernel(ChunkArgs a
 // kernels cannot share a CU -- the scan holds 138 KiB of LDS -- so the prep
 // takes CUs from the scan's chain).
 constexpr int SEG_CHUNKS = 64;
+// ... but a call of up to this many chunks is one segment: the few chunks of
+// a second one would cost a prep and a scan launch of their own, latency-bound
+// (T = 4200 / 4600 / 5000: 130.6 / 126.6 / 136.8 us in two segments, 103.3 /
+// 113.5 / 128.7 in one; from about 80 chunks the operands leave the Infinity
+// Cache and nothing is gained).
+constexpr int SEG_ONE = 80;
 // (sequence, v-head) pairs from which the local kernel runs.  Its time is the
 // longest sequence's chunk count times a chunk step, whatever the batch (up
 // to one workgroup per CU); prep + scan grows with the total chunks.
@@ -1898,11 +1987,19 @@ constexpr int LOC_MIN_PAIRS = 160;
 // 33.4-35.5 against 18.6-37.5.  (The workspace size does not depend on
 // this: a local call ignores the workspace it is given.)
 constexpr int LOC_SHORT2_PAIRS = 96;
+// (sequence, v-head) pairs scanned at once up to which chunk_scan_kernel runs:
+// its 8 workgroups per pair then have a CU each.  Up to twice that, 32 state
+// columns per workgroup, beyond, 64 (chunk_scan_cols_kernel), again a CU per
+// workgroup.  Hv = 32, 32 / 64 columns: B = 2 x T = 1038 47.8 / 52.7 us, B = 4 x
+// T = 1000 90.3 / 80.2.  A packed batch (cu_seqlens) of more sequences keeps 32
+// columns: its longest sequence, unknown here, sets the time, and a step of 32
+// columns is shorter (lengths 3000, 300, 300: 101.0 against 112.3 us with 64).
+constexpr int SCAN_ROWS_PAIRS = 32;
 
 // Workspace: the chunk table, the state carried between segments (when
 // there are several) and the scan operands of one segment.
 struct WsLayout {
-  size_t chunk_start, seqrec, carry, total;
+  size_t chunk_start, carry, total;
   size_t vh, Ut, dup;
 };
 
@@ -1912,9 +2009,7 @@ WsLayout ws_layout(int n_seqs, int64_t seg_chunks, int Hv, bool multi) {
   WsLayout l;
   size_t off = 0;
   l.chunk_start = off;
-  off = align256(off + sizeof(int32_t) * (n_seqs + 2));
-  l.seqrec = off;
-  off = align256(off + sizeof(int64_t) * SEQREC * static_cast<size_t>(n_seqs));
+  off = align256(off + sizeof(int32_t) * (n_seqs + 1));
   l.carry = off;
   if (multi) off = align256(off + sizeof(float) * static_cast<size_t>(n_seqs) * Hv * DK * DV);
   l.vh = off;
@@ -1940,9 +2035,10 @@ extern "C" size_t gdn_chunk_workspace_bytes(int32_t n_seqs, int64_t total_tokens
   using namespace gdn;
   if (n_seqs <= 0 || total_tokens < 0 || Hv <= 0 || K != DK || V != DV) return 0;
   if (static_cast<int64_t>(n_seqs) * Hv >= LOC_MIN_PAIRS) return 0;  // the local kernel keeps all in LDS
-  // Upper bound valid with or without cu_seqlens.
+  // Upper bound valid with or without cu_seqlens (a call has at most nc chunks,
+  // and at most SEG_ONE of them in a segment).
   const int64_t nc = (total_tokens + CK - 1) / CK + n_seqs;
-  return ws_layout(n_seqs, std::min<int64_t>(nc, SEG_CHUNKS), Hv, nc > SEG_CHUNKS).total;
+  return ws_layout(n_seqs, std::min<int64_t>(nc, SEG_ONE), Hv, nc > SEG_ONE).total;
 }
 
 namespace gdn {
@@ -1976,22 +2072,20 @@ int chunk_fwd(const void *q, const void *k, const void *v, int qkv_dtype,
     return fail(GDN_ERR_INVALID_ARGUMENT, "%s: q/k/v must be 16-byte aligned", name);
   const int64_t total = cu_seqlens ? static_cast<int64_t>(T) : static_cast<int64_t>(n_seqs) * T;
   const int64_t nc = max_chunks_of(n_seqs, total, cu_seqlens != nullptr, T);
-  // several sequences: the persistent scan once its (v-head, column tile)
-  // workgroups fill the CUs without spreading the sequences over the grid
   // (sequence, v-head) pairs that fill the CUs: the local kernel, one workgroup per pair
   const int64_t pairs = static_cast<int64_t>(n_seqs) * Hv;
   const int64_t longest = cu_seqlens ? (total + CK - 1) / CK : (T + CK - 1) / CK;  // chunks, or their bound
   const bool local = pairs >= LOC_MIN_PAIRS || longest == 1 || (longest == 2 && pairs >= LOC_SHORT2_PAIRS);
-  const bool persist = n_seqs > 1 && static_cast<int64_t>(Hv) * (DV / SCAN_COLS) >= SCAN_PERSIST_BLOCKS;
-  const int64_t seg = std::min<int64_t>(nc, SEG_CHUNKS);
-  const WsLayout l = ws_layout(n_seqs, seg, Hv, nc > SEG_CHUNKS);
+  const bool multi = nc > SEG_ONE;  // several segments
+  const int64_t seg = multi ? SEG_CHUNKS : nc;
+  const WsLayout l = ws_layout(n_seqs, seg, Hv, multi);
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (local) {  // one workgroup per (sequence, v-head); no workspace
     if (pairs > 0x7fffffff) return fail(GDN_ERR_INVALID_ARGUMENT, "%s: grid too large", name);
     ChunkArgs a{static_cast<const uint16_t *>(q), static_cast<const uint16_t *>(k), static_cast<const uint16_t *>(v),
                 q_stride_t, k_stride_t, v_stride_t, gate, h0, h0_idx, h0_rows, hT, hT_idx, hT_rows, o, o_dtype,
                 cu_seqlens, n_seqs, T, Hk, Hv, total, scale, l2norm_qk, static_cast<int>(std::min<int64_t>(nc, 0x7fffffff)),
-                0, 0, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
+                0, 0, 0, nullptr, nullptr, nullptr, nullptr, nullptr};
     const dim3 grid(static_cast<unsigned>(static_cast<int64_t>(n_seqs) * Hv));
     if (o_dtype == GDN_DTYPE_BF16)
       hipLaunchKernelGGL((chunk_local_kernel<true>), grid, dim3(64 * LOC_WAVES), 0, s, a);
@@ -2004,55 +2098,57 @@ int chunk_fwd(const void *q, const void *k, const void *v, int qkv_dtype,
   if (reinterpret_cast<uintptr_t>(workspace) % 256)
     return fail(GDN_ERR_WORKSPACE, "%s: workspace must be 256-byte aligned", name);
   if (nc > 65535) return fail(GDN_ERR_INVALID_ARGUMENT, "%s: %lld chunks exceed one launch", name, (long long)nc);
-  const int64_t scan_blocks = static_cast<int64_t>(persist ? 1 : n_seqs) * Hv * (DV / SCAN_COLS);
-  if (scan_blocks > 0x7fffffff) return fail(GDN_ERR_INVALID_ARGUMENT, "%s: grid too large", name);
+  // Several sequences of one length, several segments: a segment takes the
+  // same window of chunks of every sequence, so that all of them are scanned
+  // at once.  (With cu_seqlens the lengths are on the device: sequence after
+  // sequence, and a segment holds few of them.)
+  const int64_t chunks = (static_cast<int64_t>(T) + CK - 1) / CK;  // per sequence (dense)
+  const int win = multi && !cu_seqlens && n_seqs > 1 && n_seqs <= SEG_CHUNKS ? SEG_CHUNKS / n_seqs : 0;
+  const int64_t nseg = win ? (chunks + win - 1) / win : seg > 0 ? (nc + seg - 1) / seg : 0;
+  // (sequence, v-head) pairs whose chains run at the same time
+  const int64_t active = multi && !win ? Hv : pairs;
   char *ws = static_cast<char *>(workspace);
   ChunkArgs a{static_cast<const uint16_t *>(q), static_cast<const uint16_t *>(k), static_cast<const uint16_t *>(v),
               q_stride_t, k_stride_t, v_stride_t, gate, h0, h0_idx, h0_rows, hT, hT_idx, hT_rows, o, o_dtype,
-              cu_seqlens, n_seqs, T, Hk, Hv, total, scale, l2norm_qk, static_cast<int>(nc), 0, 0,
+              cu_seqlens, n_seqs, T, Hk, Hv, total, scale, l2norm_qk, static_cast<int>(nc), 0, 0, win,
               reinterpret_cast<int32_t *>(ws + l.chunk_start), reinterpret_cast<u32x4 *>(ws + l.vh),
               reinterpret_cast<float *>(ws + l.Ut),
-              reinterpret_cast<float *>(ws + l.carry), reinterpret_cast<int64_t *>(ws + l.seqrec), nullptr};
+              reinterpret_cast<float *>(ws + l.carry), nullptr};
   // q and k given per v-head (Hk == Hv): the prep checks each chunk's pairs
   // of v-heads for repeated rows and the scan reads one copy of a repeated pair
-  if (!persist && Hk == Hv && Hv % 2 == 0) a.dup = reinterpret_cast<int32_t *>(ws + l.dup);
+  if (Hk == Hv && Hv % 2 == 0) a.dup = reinterpret_cast<int32_t *>(ws + l.dup);
   auto set_segment = [&](int64_t segment) {
-    a.seg_begin = static_cast<int>(segment * seg);
+    a.seg_begin = static_cast<int>(segment * (win ? win : seg));
     a.seg_end = static_cast<int>(std::min<int64_t>((segment + 1) * seg, nc));
   };
   auto launch_prep = [&](hipStream_t st) {
     hipLaunchKernelGGL(chunk_prep_kernel, dim3(Hv, static_cast<unsigned>(seg)), dim3(256), 0, st, a);
   };
-  auto launch_scan = [&](hipStream_t st) {
-    if (persist) {
-      if (o_dtype == GDN_DTYPE_BF16)
-        hipLaunchKernelGGL((chunk_scan_persist_kernel<true>), dim3(static_cast<unsigned>(scan_blocks)),
-                           dim3(64 * SCAN_WAVES), 0, st, a);
-      else
-        hipLaunchKernelGGL((chunk_scan_persist_kernel<false>), dim3(static_cast<unsigned>(scan_blocks)),
-                           dim3(64 * SCAN_WAVES), 0, st, a);
-      return;
-    }
-    if (o_dtype == GDN_DTYPE_BF16)
-      hipLaunchKernelGGL((chunk_scan_kernel<true>), dim3(static_cast<unsigned>(scan_blocks)),
-                         dim3(64 * SCAN_WAVES), 0, st, a);
-    else
-      hipLaunchKernelGGL((chunk_scan_kernel<false>), dim3(static_cast<unsigned>(scan_blocks)),
-                         dim3(64 * SCAN_WAVES), 0, st, a);
+  auto launch_rows = [&](auto bf16) {
+    hipLaunchKernelGGL((chunk_scan_kernel<decltype(bf16)::value>), dim3(static_cast<unsigned>(pairs * (DV / SCAN_COLS))),
+                       dim3(64 * SCAN_WAVES), 0, s, a);
   };
-  // the chunk table: chunk starts for varlen, per-sequence records for the persistent scan
-  // (which computes them itself for a dense batch without slot ids)
-  if (cu_seqlens || (persist && (h0_idx || hT_idx)))
+  auto launch_cols = [&](auto nw, auto bf16) {
+    constexpr int NW = decltype(nw)::value;
+    hipLaunchKernelGGL((chunk_scan_cols_kernel<NW, decltype(bf16)::value>),
+                       dim3(static_cast<unsigned>(pairs * (DV / (16 * NW)))), dim3(64 * (NW + 2)), 0, s, a);
+  };
+  auto launch_scan = [&](auto bf16) {
+    if (active <= SCAN_ROWS_PAIRS) return launch_rows(bf16);
+    if (active <= 2 * SCAN_ROWS_PAIRS || cu_seqlens) return launch_cols(std::integral_constant<int, 2>(), bf16);
+    launch_cols(std::integral_constant<int, 4>(), bf16);
+  };
+  if (cu_seqlens)  // the chunk table
     hipLaunchKernelGGL(chunk_table_kernel, dim3(1), dim3(256), 0, s, a);
-  const int64_t nseg = seg > 0 ? (nc + seg - 1) / seg : 0;
-  if (nseg == 0) {  // only empty sequences: they still pass their state through
-    set_segment(0);
-    launch_scan(s);
-  }
-  for (int64_t kseg = 0; kseg < nseg; ++kseg) {  // segment k's scan reads the state carried from k - 1
+  // segment k's scan reads the state carried from k - 1 (no segment at all: only
+  // empty sequences, which still pass their state through)
+  for (int64_t kseg = 0; kseg < std::max<int64_t>(nseg, 1); ++kseg) {
     set_segment(kseg);
-    launch_prep(s);
-    launch_scan(s);
+    if (nseg > 0) launch_prep(s);
+    if (o_dtype == GDN_DTYPE_BF16)
+      launch_scan(std::true_type());
+    else
+      launch_scan(std::false_type());
   }
   return check_launch(name);
 }

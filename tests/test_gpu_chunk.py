@@ -563,3 +563,65 @@ def test_short_packed_batches_on_the_per_pair_kernel(lens):
     for i, n in enumerate(lens):
         if n == 0:
             assert torch.equal(s[i].cpu(), h0[i]), i
+
+
+# the column scan's dispatch: 33 to 64 pairs (32 columns per workgroup) and 65 to 159 (64), one segment and
+# windows of several (over 80 chunks), ragged ends; 160 chunks in windows of one
+@pytest.mark.parametrize("n,hv,t", [(10, 4, 200), (10, 4, 193), (16, 4, 129), (20, 4, 257), (10, 4, 700),
+                                    (20, 4, 321), (39, 4, 193), (3, 32, 2000)])
+def test_column_scan_matches_the_oracle(n, hv, t):
+    hk = hv // 2
+    gen = torch.Generator().manual_seed(1000 * n + t)
+    q, k = (torch.randn(n, t, hk, 128, generator=gen).bfloat16() for _ in range(2))
+    v = torch.randn(n, t, hv, 128, generator=gen).bfloat16()
+    c = dict(q=q, k=k, v=v, g=-torch.rand(n, t, hv, generator=gen), beta=torch.rand(n, t, hv, generator=gen))
+    h0 = torch.randn(n, hv, 128, 128, generator=gen) * 0.1
+    print(f"n={n} hv={hv} t={t}", flush=True)
+    o, s = run_chunk(c, h0)
+    sel = list(range(n)) if n * hv < 64 else [0, n // 2, n - 1]  # (the oracle on a few sequences of the large ones)
+    heads = slice(0, hv) if hv < 32 else slice(14, 18)
+    kh = slice(heads.start // 2, (heads.stop + 1) // 2)
+    sub = {x: c[x][sel][:, :, kh if x in "qk" else heads] for x in c}
+    o_ref, s_ref = oracle_chunk(sub, h0[sel][:, heads])
+    assert np.abs(np64(o)[sel][:, :, heads] - o_ref).max() < O_TOL
+    assert gdn.state_rel_err(np64(s)[sel][:, heads], s_ref) < S_TOL
+    # q and k repeated to the v-heads: the odd heads read their partner's copy, the same bits
+    rep = dict(c, q=q.repeat_interleave(2, 2), k=k.repeat_interleave(2, 2))
+    o2, s2 = run_chunk(rep, h0)
+    assert torch.equal(o2, o) and torch.equal(s2, s)
+
+
+@pytest.mark.parametrize("lens,hv", [([200, 0, 64, 65, 1, 0, 130, 17, 63, 128], 4), ([100] * 17, 4),
+                                     ([900, 0, 3000, 64, 2000], 8), ([5200], 2)])
+def test_column_scan_packed_on_a_slot_pool(lens, hv):
+    """Packed batches of 33 or more pairs (and, multi-segment, of several sequences) in place on a slot pool
+    with a repeated and a negative id, sequence by sequence."""
+    n, hk, gen = len(lens), hv // 2, torch.Generator().manual_seed(sum(lens))
+    t = sum(lens)
+    cu = torch.tensor([0] + list(np.cumsum(lens)), dtype=torch.int32)
+    q, k = (torch.randn(1, t, hk, 128, generator=gen).bfloat16() for _ in range(2))
+    v = torch.randn(1, t, hv, 128, generator=gen).bfloat16()
+    c = dict(q=q, k=k, v=v, g=-torch.rand(1, t, hv, generator=gen), beta=torch.rand(1, t, hv, generator=gen))
+    slots = torch.randperm(n + 3, generator=gen)[:n]
+    if n > 3:
+        slots[2], slots[3] = slots[0], -1
+    pool = torch.randn(n + 3, hv, 128, 128, generator=gen) * 0.1
+    p = pool.to(DEV)
+    args = [c[x].to(DEV) for x in ("q", "k", "v", "g", "beta")]
+    o, _ = chunk_gated_delta_rule(*args, initial_state=p, ssm_state_indices=slots.to(DEV), inplace_final_state=True,
+                                  use_qk_l2norm_in_kernel=True, cu_seqlens=cu.to(DEV))
+    seen = set()
+    for i, ln in enumerate(lens):
+        sl = int(slots[i])
+        own = sl >= 0 and sl not in seen
+        seen.add(sl)
+        h0 = pool[sl:sl + 1] if own else torch.zeros(1, hv, 128, 128)
+        if ln:
+            o_ref, s_ref = oracle_chunk({x: c[x][:, cu[i]:cu[i + 1]] for x in c}, h0)
+            assert np.abs(np64(o)[:, cu[i]:cu[i + 1]] - o_ref).max() < O_TOL, i
+        else:
+            s_ref = h0.numpy()
+        if own:
+            assert gdn.state_rel_err(np64(p[sl:sl + 1]), s_ref) < S_TOL, i
+    for sl in set(range(n + 3)) - set(slots.tolist()):
+        assert torch.equal(p[sl].cpu(), pool[sl])
