@@ -5,6 +5,9 @@
 Each csrc/*.hip file is compiled to an object with hipcc, then linked into
 engine/kernels/libgdn_mi355x.so next to the ctypes loader.  Packed fp32
 instructions are disabled for all device code (-packed-fp32-ops).
+csrc/gdn_host.cpp (the native host path, no device code) becomes the
+extension module engine/kernels/_gdn_host.so, built against the installed
+torch.
 """
 from __future__ import annotations
 
@@ -22,6 +25,7 @@ INCLUDE = os.path.join(REPO, "include")
 BUILD = os.path.join(PKG, "_build")
 LIB_NAME = "libgdn_mi355x.so"
 LIB_PATH = os.path.join(PKG, "engine", "kernels", LIB_NAME)
+HOST_PATH = os.path.join(PKG, "engine", "kernels", "_gdn_host.so")
 ARCH = "gfx950"
 
 
@@ -65,13 +69,38 @@ def _compile(src: str, verbose: bool) -> str:
     return obj
 
 
+def _build_host(verbose: bool) -> None:
+    """The host extension: plain C++ against torch's and HIP's headers."""
+    import sysconfig
+
+    import torch
+    troot = os.path.dirname(torch.__file__)
+    rocm = os.path.dirname(os.path.dirname(hipcc()))
+    tmp = HOST_PATH + ".tmp"
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
+           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}",
+           "-I", INCLUDE, "-I", os.path.join(troot, "include"),
+           "-I", os.path.join(troot, "include", "torch", "csrc", "api", "include"),
+           "-I", os.path.join(rocm, "include"), "-I", sysconfig.get_paths()["include"],
+           os.path.join(CSRC, "gdn_host.cpp"), "-o", tmp, "-L", os.path.join(troot, "lib"),
+           "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"host extension failed:\n{res.stdout}\n{res.stderr}")
+    os.replace(tmp, HOST_PATH)
+
+
 def build(jobs: int | None = None, verbose: bool = False) -> str:
     """Compile every kernel source and link the shared library; returns its path."""
     os.makedirs(BUILD, exist_ok=True)
     srcs = sources()
     jobs = jobs or min(len(srcs), max(1, (os.cpu_count() or 2) // 2), 8)
-    with cf.ThreadPoolExecutor(max_workers=jobs) as ex:
+    with cf.ThreadPoolExecutor(max_workers=jobs + 1) as ex:
+        host = ex.submit(_build_host, verbose)
         objs = list(ex.map(lambda s: _compile(s, verbose), srcs))
+        host.result()
     tmp = LIB_PATH + ".tmp"
     # -z defs: an unresolved symbol (e.g. a kernel whose host stub was not
     # emitted) fails the link instead of the library's load

@@ -123,6 +123,13 @@ SIGNATURES = {
 }
 
 _LIB: Optional[ctypes.CDLL] = None
+_HOST = None
+
+HOST_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "_gdn_host.so")
+# the entry points that the host extension calls, in its order (csrc/gdn_host.cpp: Entries)
+HOST_ENTRIES = ("gdn_last_error_string", "gdn_recurrent_fwd", "gdn_recurrent_fwd_gated", "gdn_chunk_fwd",
+                "gdn_chunk_fwd_gated", "gdn_chunk_workspace_bytes", "gdn_rmsnorm_gated_fwd", "gdn_in_proj_decode",
+                "gdn_out_proj_workspace_bytes", "gdn_out_proj_decode", "causal_conv1d_fwd")
 
 
 def load(path: str = LIB_PATH) -> ctypes.CDLL:
@@ -146,6 +153,30 @@ def load(path: str = LIB_PATH) -> ctypes.CDLL:
     return lib
 
 
+def host():
+    """The host extension (csrc/gdn_host.cpp), bound to the loaded library:
+    its functions run a wrapper's regular call natively, or return None for
+    the wrapper to go its general way.  Raises if it is missing."""
+    return _HOST if _HOST is not None else _load_host()
+
+
+def _load_host():
+    global _HOST
+    lib = load()
+    if not os.path.exists(HOST_PATH):
+        raise RuntimeError(
+            f"{os.path.basename(HOST_PATH)} not found at {HOST_PATH}; build it with "
+            "`python paris-hackathon-2026-inference_amd/build_lib.py`")
+    import importlib.machinery
+    import importlib.util
+    loader = importlib.machinery.ExtensionFileLoader("_gdn_host", HOST_PATH)
+    mod = importlib.util.module_from_spec(importlib.util.spec_from_loader("_gdn_host", loader))
+    loader.exec_module(mod)
+    mod.bind(*(ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in HOST_ENTRIES))
+    _HOST = mod
+    return mod
+
+
 def check(status: int, what: str) -> None:
     if status != 0:
         msg = load().gdn_last_error_string().decode(errors="replace")
@@ -157,7 +188,7 @@ def ptr(t: Optional[torch.Tensor]) -> Optional[int]:
 
 
 def stream_of(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 
 def require_gpu(*tensors: Optional[torch.Tensor]) -> torch.device:

@@ -79,6 +79,21 @@ def causal_conv1d_fn(
       * ``return_final_states`` / ``final_states_out`` [N, C, S]: final windows.
     Returns y (same layout as x), or ``(y, final_states)``.
     """
+    return _conv1d_fn(x, weight, bias, activation, cu_seqlens, initial_states, conv_states, cache_indices,
+                      has_initial_state, return_final_states, final_states_out)
+
+
+def _conv1d_fn(x, weight, bias, activation, cu_seqlens=None, initial_states=None, conv_states=None, cache_indices=None,
+               has_initial_state=None, return_final_states=False, final_states_out=None, read_indices=None):
+    """:func:`causal_conv1d_fn`; ``read_indices`` [N] int64 in the place of
+    ``has_initial_state``: the pool rows whose windows are the history
+    (negative: zeros), decided by the caller."""
+    if (initial_states is None and has_initial_state is None and not return_final_states and final_states_out is None
+            and activation in (None, False, "silu", "swish", True)):
+        done = _lib.host().conv(x, weight, bias, activation in ("silu", "swish", True), conv_states, cache_indices,
+                                read_indices, cu_seqlens)
+        if done is not None:
+            return done
     dev = _lib.require_gpu(x, weight, bias, initial_states, conv_states, final_states_out)
     dt = x.dtype
     if dt not in (torch.bfloat16, torch.float16, torch.float32):
@@ -113,6 +128,8 @@ def causal_conv1d_fn(
             if idx is not None:  # a repeated slot id neither reads nor writes: decide it on the unmasked ids
                 has = has & ~(base[:, None] == base[None, :]).tril(-1).any(dim=1)
             in_idx = torch.where(has, base, torch.full_like(base, -1))
+        elif read_indices is not None:
+            in_idx = _lib.as_index(read_indices, dev)
     if initial_states is not None:
         if initial_states.shape[:2] != (n_seqs, c):
             raise ValueError(f"initial_states must be [{n_seqs}, {c}, S]")

@@ -76,6 +76,11 @@ def chunk_gated_delta_rule(
     last_recurrent_state [N, Hv, K, V] fp32 or None)`` as the reference does
     (delta_rule.py:366-374).
     """
+    if chunk_size == CHUNK_SIZE and has_initial_state is None:
+        done = _lib.host().chunk(query, key, value, g, beta, None, None, scale, use_qk_l2norm_in_kernel, initial_state,
+                                 ssm_state_indices, cu_seqlens, inplace_final_state, output_final_state, None)
+        if done is not None:
+            return done
     b, t, hv = value.shape[0], value.shape[1], value.shape[2]
     _lib.require_gpu(g, beta)
     g32, _ = _lib.per_token(g.to(torch.float32), b, t, hv, "g")
@@ -111,6 +116,23 @@ def chunk_gated_delta_rule_from_projections(
     ``A_log``, ``dt_bias`` ``[Hv]``): beta = sigmoid(b),
     g = -exp(A_log) * softplus(a + dt_bias), the glue of HF's layer forward
     (transformers modeling_qwen3_5_moe.py:495-497)."""
+    return _from_projections(query, key, value, a, b, A_log, dt_bias, initial_state, output_final_state,
+                             use_qk_l2norm_in_kernel, cu_seqlens, scale, ssm_state_indices, inplace_final_state,
+                             has_initial_state)
+
+
+def _from_projections(query, key, value, a, b, A_log, dt_bias, initial_state, output_final_state,
+                      use_qk_l2norm_in_kernel, cu_seqlens, scale, ssm_state_indices, inplace_final_state,
+                      has_initial_state=None, read_indices=None):
+    """:func:`chunk_gated_delta_rule_from_projections`; ``read_indices`` [N]
+    int64 in the place of ``has_initial_state``: the pool rows to start from
+    (negative: a zero state), decided by the caller."""
+    if has_initial_state is None:
+        done = _lib.host().chunk(query, key, value, a, b, _lib.f32_vector(A_log), _lib.f32_vector(dt_bias), scale,
+                                 use_qk_l2norm_in_kernel, initial_state, ssm_state_indices, cu_seqlens,
+                                 inplace_final_state, output_final_state, read_indices)
+        if done is not None:
+            return done
     bsz, t, hv = value.shape[0], value.shape[1], value.shape[2]
     _lib.require_gpu(a, b, A_log, dt_bias)
     if a.dtype not in _lib.GDN_DTYPE:
@@ -129,14 +151,14 @@ def chunk_gated_delta_rule_from_projections(
     keep = (ax, bx, alog, dtb)  # alive until the launch is enqueued
     out = _chunk(query, key, value, gates, CHUNK_SIZE, initial_state, output_final_state,
                  use_qk_l2norm_in_kernel, cu_seqlens, scale, ssm_state_indices, inplace_final_state,
-                 has_initial_state)
+                 has_initial_state, read_indices)
     del keep
     return out
 
 
 def _chunk(query, key, value, gates, chunk_size, initial_state, output_final_state,
            use_qk_l2norm_in_kernel, cu_seqlens, scale, ssm_state_indices, inplace_final_state,
-           has_initial_state=None):
+           has_initial_state=None, read_indices=None):
     """Shared body: shape checks, state / workspace plumbing and the launch.
     ``gates`` = (entry point, its gate arguments)."""
     if int(chunk_size) <= 0:
@@ -198,6 +220,8 @@ def _chunk(query, key, value, gates, chunk_size, initial_state, output_final_sta
             rep = (rows[:, None] == rows[None, :]).tril(-1).any(dim=1)
             has = has & ~rep
         h0_idx = torch.where(has, rows, torch.full_like(rows, -1))
+    elif read_indices is not None:
+        h0_idx = _lib.as_index(read_indices, dev)
     if output_final_state and not inplace_final_state:
         final = hT = torch.empty((n_seqs, hv, dk, dv), dtype=torch.float32, device=dev)
         hT_idx = None

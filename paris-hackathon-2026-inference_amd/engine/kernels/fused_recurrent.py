@@ -54,6 +54,10 @@ def fused_recurrent_gated_delta_rule(
 
     Returns ``(o [B, T, Hv, V] in q's dtype, final_state or None)``.
     """
+    done = _lib.host().recurrent(q, k, v, g, beta, None, None, scale, use_qk_l2norm_in_kernel, initial_state,
+                                 ssm_state_indices, cu_seqlens, inplace_final_state, output_final_state, snapshots)
+    if done is not None:
+        return done
     _lib.require_gpu(q, g, beta)
     if beta is None:
         beta = torch.ones_like(g)
@@ -90,6 +94,11 @@ def fused_recurrent_gated_delta_rule_from_projections(
     ``[B, T, Hv]``, ``A_log``, ``dt_bias`` ``[Hv]``; beta = sigmoid(b),
     g = -exp(A_log) * softplus(a + dt_bias) (transformers
     modeling_qwen3_5_moe.py:495-497)."""
+    done = _lib.host().recurrent(q, k, v, a, b, _lib.f32_vector(A_log), _lib.f32_vector(dt_bias), scale,
+                                 use_qk_l2norm_in_kernel, initial_state, ssm_state_indices, cu_seqlens,
+                                 inplace_final_state, output_final_state, snapshots)
+    if done is not None:
+        return done
     bsz, t, hv = v.shape[0], v.shape[1], v.shape[2]
     _lib.require_gpu(q, a, b, A_log, dt_bias)
     if a.dtype not in _lib.GDN_DTYPE:

@@ -36,8 +36,8 @@ from typing import Optional
 import torch
 
 from . import _lib
-from .causal_conv1d import causal_conv1d_fn, causal_conv1d_update
-from .delta_rule import chunk_gated_delta_rule_from_projections
+from .causal_conv1d import _conv1d_fn, causal_conv1d_fn, causal_conv1d_update
+from .delta_rule import _from_projections, chunk_gated_delta_rule_from_projections
 from .fused_recurrent import fused_recurrent_gated_delta_rule_from_projections
 from .in_proj import OUT_PROJ_MAX_M, fused_in_proj_supported, fused_out_proj_supported, gdn_in_proj_decode, gdn_out_proj_decode
 
@@ -51,6 +51,10 @@ def rms_norm_gated(x: torch.Tensor, z: torch.Tensor, weight: torch.Tensor, eps: 
     (default x's).  x, z ``[..., H, D]``; rows of a token may be strided
     views (token stride a multiple of 8 elements).  Replaces HF's
     RMSNormGated (transformers modeling_qwen3_5_moe.py:169-185)."""
+    if out_dtype is None:
+        done = _lib.host().rms_norm(x, z, weight, eps)
+        if done is not None:
+            return done
     dev = _lib.require_gpu(x, z, weight)
     if x.shape != z.shape:
         raise ValueError(f"x{tuple(x.shape)} and z{tuple(z.shape)} differ")
@@ -81,19 +85,38 @@ def rms_norm_gated(x: torch.Tensor, z: torch.Tensor, weight: torch.Tensor, eps: 
     return y.view(x.shape)
 
 
+def _weight_bias(lin) -> tuple:
+    """A projection's weight and bias, from its parameter table where they
+    are plain parameters (an ``nn.Module`` attribute costs the interpreter a
+    microsecond)."""
+    table = lin._parameters
+    w = table.get("weight")
+    return (lin.weight if w is None else w), (table["bias"] if "bias" in table else lin.bias)
+
+
+def _projections(self) -> list:
+    mods = self._modules
+    return [mods[n] if n in mods else getattr(self, n)
+            for n in ("in_proj_qkv", "in_proj_z", "in_proj_b", "in_proj_a", "conv1d")]
+
+
 def _fused_decode_fits(self, hidden_states: torch.Tensor, conv_state: torch.Tensor) -> bool:
     """Whether this one-token step can take :func:`gdn_in_proj_decode`: bf16
     bias-free projections of a supported shape and a bf16 [rows, C, 4] window
     pool."""
-    lins = (self.in_proj_qkv, self.in_proj_z, self.in_proj_b, self.in_proj_a)
     if hidden_states.dtype != torch.bfloat16 or hidden_states.shape[1] != 1:
         return False
-    if any(l.bias is not None or l.weight.dtype != torch.bfloat16 for l in lins):
+    *lins, conv = _projections(self)
+    n = []
+    for lin in lins:
+        w, bias = _weight_bias(lin)
+        if bias is not None or w.dtype != torch.bfloat16:
+            return False
+        n.append(w.shape[0])
+    conv_w = _weight_bias(conv)[0]
+    if conv_w.dtype != torch.bfloat16 or self.activation not in ("silu", "swish", None):
         return False
-    if self.conv1d.weight.dtype != torch.bfloat16 or self.activation not in ("silu", "swish", None):
-        return False
-    n = [l.weight.shape[0] for l in lins]
-    if not fused_in_proj_supported(hidden_states.shape[-1], *n, self.conv1d.weight.shape[-1]):
+    if not fused_in_proj_supported(hidden_states.shape[-1], *n, conv_w.shape[-1]):
         return False
     return (conv_state.dtype == torch.bfloat16 and conv_state.dim() == 3 and conv_state.is_contiguous()
             and tuple(conv_state.shape[1:]) == (n[0], 4))
@@ -101,13 +124,11 @@ def _fused_decode_fits(self, hidden_states: torch.Tensor, conv_state: torch.Tens
 
 def _fused_decode(self, hidden_states: torch.Tensor, conv_state: torch.Tensor,
                   slots: Optional[torch.Tensor]) -> tuple[torch.Tensor, ...]:
-    """(mixed_qkv after the conv [B, 1, C], z [B, 1, Hv*V], b, a [B, 1, Hv])
-    of a one-token step, conv windows advanced in place."""
-    batch_size = hidden_states.shape[0]
-    y, z, b, a = gdn_in_proj_decode(hidden_states.reshape(batch_size, -1), self.in_proj_qkv.weight,
-                                    self.in_proj_z.weight, self.in_proj_b.weight, self.in_proj_a.weight,
-                                    self.conv1d.weight, self.conv1d.bias, conv_state, slots, self.activation)
-    return tuple(t.view(batch_size, 1, -1) for t in (y, z, b, a))
+    """(mixed_qkv after the conv [B, C], z [B, Hv*V], b, a [B, Hv]) of a
+    one-token step, conv windows advanced in place."""
+    *lins, conv = _projections(self)
+    return gdn_in_proj_decode(hidden_states, *(_weight_bias(lin)[0] for lin in lins), *_weight_bias(conv), conv_state,
+                              slots, self.activation)
 
 
 def _out_proj_fits(self, out: torch.Tensor) -> bool:
@@ -115,15 +136,17 @@ def _out_proj_fits(self, out: torch.Tensor) -> bool:
     one token per row, at most OUT_PROJ_MAX_M rows, a plain bias-free bf16
     ``nn.Linear`` of a supported shape."""
     lin = self.out_proj
-    return (type(lin) is torch.nn.Linear and out.shape[1] == 1 and out.shape[0] <= OUT_PROJ_MAX_M
-            and out.dtype == torch.bfloat16 and lin.bias is None and lin.weight.dtype == torch.bfloat16
-            and fused_out_proj_supported(lin.weight.shape[1], lin.weight.shape[0]))
+    if type(lin) is not torch.nn.Linear or out.shape[1] != 1 or out.shape[0] > OUT_PROJ_MAX_M:
+        return False
+    w, bias = _weight_bias(lin)
+    return (out.dtype == torch.bfloat16 and bias is None and w.dtype == torch.bfloat16
+            and fused_out_proj_supported(w.shape[1], w.shape[0]))
 
 
 def _out_proj(self, out: torch.Tensor) -> torch.Tensor:
     """``self.out_proj(out)`` for ``out`` [B, L, Hv*V]; decode rows through the kernel."""
     if _out_proj_fits(self, out):
-        return gdn_out_proj_decode(out, self.out_proj.weight)
+        return gdn_out_proj_decode(out, _weight_bias(self.out_proj)[0])
     return self.out_proj(out)
 
 
@@ -145,7 +168,8 @@ def gated_delta_net_forward(self, hidden_states: torch.Tensor, cache_params=None
     decode_step = use_precomputed_states and seq_len == 1 and not layer.record_past
     if decode_step and layer.conv_states[0].shape[0] == batch_size and _fused_decode_fits(
             self, hidden_states, layer.conv_states[0]):
-        mixed_qkv, z, b, a = _fused_decode(self, hidden_states, layer.conv_states[0], None)
+        projected = _fused_decode(self, hidden_states, layer.conv_states[0], None)
+        mixed_qkv, z, b, a = (t.view(batch_size, 1, -1) for t in projected)
     else:
         mixed_qkv = self.in_proj_qkv(hidden_states).transpose(1, 2)
         z = self.in_proj_z(hidden_states)
@@ -196,6 +220,21 @@ def gated_delta_net_forward(self, hidden_states: torch.Tensor, cache_params=None
 _RECURRENT_MAX_T = 16
 
 
+def _native_core(self, qkv: torch.Tensor, z: torch.Tensor, b: torch.Tensor, a: torch.Tensor, slots: torch.Tensor,
+                 rec_pool: torch.Tensor) -> Optional[torch.Tensor]:
+    """Between a one-token step's projections, in one native call: the
+    recurrence on the pools and the gated norm (the kernels of the general way
+    below, in its order), ``[B, 1, Hv*V]``; None where its form is not the
+    regular one."""
+    params, norm = self._parameters, self._modules.get("norm")
+    alog, dtb = params.get("A_log"), params.get("dt_bias")
+    if alog is None or dtb is None or norm is None:
+        return None
+    return _lib.host().core_decode(qkv, z, b, a, slots, self.key_dim, self.value_dim, self.head_k_dim, self.head_v_dim,
+                                   _lib.f32_vector(alog), _lib.f32_vector(dtb), rec_pool,
+                                   norm._parameters.get("weight"), norm.variance_epsilon)
+
+
 def _forward_on_pools(self, hidden_states: torch.Tensor, pools, attention_mask: Optional[torch.Tensor]) -> torch.Tensor:
     """The layer forward on slot pools (:class:`engine.runtime.slot_pools.GDNSlotPools`):
     conv and recurrent state are read from and written to ``pool[slot]`` by
@@ -205,8 +244,8 @@ def _forward_on_pools(self, hidden_states: torch.Tensor, pools, attention_mask: 
     the snapshots and conv history that ``pools.commit_verify`` rolls back to."""
     hf = sys.modules[type(self).__module__]
     hidden_states = hf.apply_mask_to_padding_states(hidden_states, attention_mask)
-    batch_size, seq_len, _ = hidden_states.shape
     conv_pool, rec_pool = pools.layer(self.layer_idx)
+    batch_size, seq_len, _ = hidden_states.shape
     slots = pools.slots()
     if slots.numel() != batch_size:
         raise ValueError(f"pools bound for {slots.numel()} rows, forward has {batch_size}")
@@ -220,7 +259,11 @@ def _forward_on_pools(self, hidden_states: torch.Tensor, pools, attention_mask: 
     # (which keep no snapshots)
     step = pools.decode and seq_len == 1 and not verify
     if step and _fused_decode_fits(self, hidden_states, conv_pool):
-        mixed_qkv, z, b, a = _fused_decode(self, hidden_states, conv_pool, slots)
+        projected = _fused_decode(self, hidden_states, conv_pool, slots)
+        out = _native_core(self, *projected, slots, rec_pool)
+        if out is not None:
+            return _out_proj(self, out)
+        mixed_qkv, z, b, a = (t.view(batch_size, 1, -1) for t in projected)
     else:
         mixed_qkv = self.in_proj_qkv(hidden_states).transpose(1, 2)  # [B, conv_dim, L]
         z = self.in_proj_z(hidden_states)
@@ -233,9 +276,8 @@ def _forward_on_pools(self, hidden_states: torch.Tensor, pools, attention_mask: 
         else:
             if verify:
                 pools.record_conv(self.layer_idx, mixed_qkv)
-            mixed_qkv = causal_conv1d_fn(mixed_qkv, conv_w, self.conv1d.bias, activation=self.activation,
-                                         conv_states=conv_pool, cache_indices=slots,
-                                         has_initial_state=pools.has_state())
+            mixed_qkv = _conv1d_fn(mixed_qkv, conv_w, self.conv1d.bias, self.activation, conv_states=conv_pool,
+                                   cache_indices=slots, read_indices=pools.read_slots())
         mixed_qkv = mixed_qkv.transpose(1, 2)
     query, key, value = torch.split(mixed_qkv, [self.key_dim, self.key_dim, self.value_dim], dim=-1)
     query = query.reshape(batch_size, seq_len, -1, self.head_k_dim)
@@ -247,10 +289,8 @@ def _forward_on_pools(self, hidden_states: torch.Tensor, pools, attention_mask: 
             use_qk_l2norm_in_kernel=True, ssm_state_indices=slots, inplace_final_state=True,
             snapshots=pools.snapshots(self.layer_idx) if verify else None)
     else:
-        core, _ = chunk_gated_delta_rule_from_projections(
-            query, key, value, a, b, self.A_log, self.dt_bias, initial_state=rec_pool,
-            use_qk_l2norm_in_kernel=True, ssm_state_indices=slots, inplace_final_state=True,
-            has_initial_state=pools.has_state())
+        core, _ = _from_projections(query, key, value, a, b, self.A_log, self.dt_bias, rec_pool, False, True, None,
+                                    None, slots, True, read_indices=pools.read_slots())
 
     z = z.reshape(batch_size, seq_len, -1, self.head_v_dim)
     out = rms_norm_gated(core, z, self.norm.weight, self.norm.variance_epsilon)

@@ -54,6 +54,11 @@ def gdn_in_proj_decode(hidden: torch.Tensor, w_qkv: torch.Tensor, w_z: torch.Ten
     ``[0, rows)`` (the engine's padding rows) read a zero window and write
     nothing.  ``activation``: ``"silu"`` or None, as ``causal_conv1d_update``.
     """
+    if activation in (None, False, "silu", "swish", True):
+        done = _lib.host().in_proj(hidden, w_qkv, w_z, w_b, w_a, conv_weight, conv_bias, conv_state,
+                                   conv_state_indices, activation in ("silu", "swish", True))
+        if done is not None:
+            return done
     dev = _lib.require_gpu(hidden, w_qkv, w_z, w_b, w_a, conv_weight, conv_state)
     x = hidden.reshape(-1, hidden.shape[-1]) if hidden.dim() == 3 else hidden
     if x.dim() != 2 or x.dtype != torch.bfloat16:
@@ -108,6 +113,9 @@ def gdn_out_proj_decode(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     weight the ``nn.Linear`` weight ``[N, K]`` bf16; returns ``[M, N]`` bf16
     (``[M, 1, N]`` for a 3-d x).  The partial sums over K are added in a
     fixed order, so the result does not depend on scheduling."""
+    done = _lib.host().out_proj(x, weight)
+    if done is not None:
+        return done
     dev = _lib.require_gpu(x, weight)
     x2 = x.reshape(-1, x.shape[-1]) if x.dim() == 3 else x
     if x2.dim() != 2 or x2.dtype != torch.bfloat16:

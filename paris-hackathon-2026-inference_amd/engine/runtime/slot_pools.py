@@ -69,6 +69,7 @@ class GDNSlotPools:
         self.max_batch = int(max_batch or self.num_slots)
         self._slots = torch.full((self.max_batch,), GDN_PAD_SLOT, dtype=torch.int64, device=self.device)
         self._has_state = torch.zeros(self.max_batch, dtype=torch.bool, device=self.device)
+        self._read = torch.full((self.max_batch,), GDN_PAD_SLOT, dtype=torch.int64, device=self.device)
         self.batch_size = 0
         self.decode = False
         self.verify_tokens = 0
@@ -118,6 +119,10 @@ class GDNSlotPools:
         self._slots[:b].copy_(torch.where(ok, ids, torch.full_like(ids, GDN_PAD_SLOT)))
         self._slots[b:].fill_(GDN_PAD_SLOT)
         self._has_state.fill_(not is_prefill)
+        if is_prefill:
+            self._read.fill_(GDN_PAD_SLOT)
+        else:
+            self._read.copy_(self._slots)
         self.batch_size = b
         self.decode = not is_prefill
         if verify_tokens:
@@ -131,6 +136,12 @@ class GDNSlotPools:
     def has_state(self) -> torch.Tensor:
         """Per row: continue from the slot's state (decode) or start from zero (prefill)."""
         return self._has_state[: self.batch_size]
+
+    def read_slots(self) -> torch.Tensor:
+        """Slot ids the bound batch's rows start from (a view of a persistent
+        buffer): the rows' own slots in a decode step, ``GDN_PAD_SLOT`` (a zero
+        state and window) in a prefill."""
+        return self._read[: self.batch_size]
 
     def layer(self, layer_idx: int) -> Tuple[torch.Tensor, torch.Tensor]:
         """(conv pool, recurrent pool) of a GDN layer."""
