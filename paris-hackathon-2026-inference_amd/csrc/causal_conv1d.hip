@@ -21,8 +21,12 @@ namespace {
 
 constexpr int CPT = 8;         // channels per thread
 constexpr int CONV_NT = 256;   // threads per workgroup
-// Tokens per workgroup tile: 32 when a 64-token grid would leave CUs
-// without a workgroup (short inputs), else the longest of 64, 56 and 48
+// Tokens per workgroup tile: 8 or 16 while that grid is one round over the CUs
+// (short inputs are bound by a tile's serial walk: 100 / 333 / 512 tokens of
+// 8192 channels with tiles of 8 / 16 / 32 8.3 / 9.6 / 12.5, 9.0 / 11.0 / 13.1
+// and 9.9 / 11.3 / 14.0 us; 1,024 tokens with 16 / 32 12.8 / 15.1; a second round
+// costs more than it saves: 750 tokens with 8 14.7 against 12.4 with 16), 32 when
+// a 64-token grid would leave CUs without a workgroup, else the longest of 64, 56 and 48
 // whose busiest CU streams the fewest tokens, ceil(workgroups / CUs) x tile:
 // a long tile halves the re-read 3-token halo against 32 and keeps more loads
 // in flight per thread, and a grid that is not a whole number of rounds over
@@ -49,8 +53,7 @@ template <> struct Vec8<uint16_t> {
     uint32_t w[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-      w[i] = static_cast<uint32_t>(f32_to_bf16_bits(x[2 * i])) |
-             (static_cast<uint32_t>(f32_to_bf16_bits(x[2 * i + 1])) << 16);
+      w[i] = f32_to_bf16_pair(x[2 * i], x[2 * i + 1]);
     *reinterpret_cast<uint4 *>(p) = make_uint4(w[0], w[1], w[2], w[3]);
   }
 };
@@ -376,11 +379,15 @@ template <typename T, int SL>
 int launch_fwd(const ConvArgs &a, hipStream_t s) {
   const unsigned gx = (a.C / CPT + CONV_NT - 1) / CONV_NT;
   if (a.total > 0) {
+    auto workgroups = [&](int64_t tile) { return gx * ((a.total + tile - 1) / tile); };
     auto busiest = [&](int64_t tile) {  // tokens streamed by the CU with the most workgroups
-      const int64_t n = gx * ((a.total + tile - 1) / tile);
-      return (n + CONV_CUS - 1) / CONV_CUS * tile;
+      return (workgroups(tile) + CONV_CUS - 1) / CONV_CUS * tile;
     };
-    if (gx * ((a.total + TILE_LONG - 1) / TILE_LONG) < CONV_CUS) {
+    if (workgroups(8) <= CONV_CUS) {
+      launch_tiles<T, SL, 8>(a, gx, s);
+    } else if (workgroups(16) <= CONV_CUS) {
+      launch_tiles<T, SL, 16>(a, gx, s);
+    } else if (workgroups(TILE_LONG) < CONV_CUS) {
       launch_tiles<T, SL, TILE_SHORT>(a, gx, s);
     } else {
       int tile = TILE_LONG;

@@ -103,18 +103,13 @@ __device__ __forceinline__ bf16x8 pack_hi(f32x4 a, f32x4 b) {
   }
   return r;
 }
-typedef __attribute__((ext_vector_type(2))) float f32x2;
-typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
-__device__ __forceinline__ uint32_t cvt2(float a, float b) {  // one v_cvt_pk_bf16_f32
-  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{a, b}), bf16x2));
-}
 // x as bf16 hi + lo, converted in pairs (hi's values are its bits moved up)
 __device__ __forceinline__ void split4(f32x4 x, u32x2 &hi, u32x2 &lo) {
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
-    const uint32_t h = cvt2(x[2 * i], x[2 * i + 1]);
+    const uint32_t h = f32_to_bf16_pair(x[2 * i], x[2 * i + 1]);
     hi[i] = h;
-    lo[i] = cvt2(x[2 * i] - __uint_as_float(h << 16), x[2 * i + 1] - __uint_as_float(h & 0xffff0000u));
+    lo[i] = f32_to_bf16_pair(x[2 * i] - __uint_as_float(h << 16), x[2 * i + 1] - __uint_as_float(h & 0xffff0000u));
   }
 }
 __device__ __forceinline__ void pack_hilo(f32x4 a, f32x4 b, bf16x8 &hi, bf16x8 &lo) {

@@ -39,11 +39,17 @@ __device__ __forceinline__ float bf16_bits_to_f32(uint16_t b) {
   return __uint_as_float(static_cast<uint32_t>(b) << 16);
 }
 
-// Round-to-nearest-even fp32 -> bf16 bits (inputs here are finite).
+// Round-to-nearest-even fp32 -> bf16 bits, one value or two (the first in the
+// low half), by the hardware conversion (v_cvt_pk_bf16_f32: one instruction
+// for both; the integer form took four per value: the conv of 333 / 1,024
+// tokens of 8192 channels 14.5 / 16.0 -> 13.2 / 14.9 us, of 4,096 and more 1%).
+typedef __attribute__((ext_vector_type(2))) float f32x2_t;
+typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2_t;
 __device__ __forceinline__ uint16_t f32_to_bf16_bits(float f) {
-  uint32_t u = __float_as_uint(f);
-  u += 0x7fffu + ((u >> 16) & 1u);
-  return static_cast<uint16_t>(u >> 16);
+  return __builtin_bit_cast(uint16_t, static_cast<__bf16>(f));
+}
+__device__ __forceinline__ uint32_t f32_to_bf16_pair(float lo, float hi) {
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2_t{lo, hi}), bf16x2_t));
 }
 
 __device__ __forceinline__ float load_elem(const void *p, int64_t i, int dt) {

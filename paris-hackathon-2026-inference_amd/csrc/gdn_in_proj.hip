@@ -111,7 +111,7 @@ __device__ __forceinline__ f32x4_t mfma16(u32x4_t a, u32x4_t b, f32x4_t c) {
 __device__ __forceinline__ float silu_f(float v) { return v / (1.f + expf(-v)); }
 
 __device__ __forceinline__ uint32_t pack2(float lo, float hi) {
-  return static_cast<uint32_t>(f32_to_bf16_bits(lo)) | (static_cast<uint32_t>(f32_to_bf16_bits(hi)) << 16);
+  return f32_to_bf16_pair(lo, hi);
 }
 
 // This wave's weights, KS k-steps of its part: lane (r, g) of k-step s

@@ -65,15 +65,13 @@ __device__ __forceinline__ void store8(void *p, int64_t i, int dt, const float (
     u32x4 a;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      uint32_t lo, hi;
       if (dt == GDN_DTYPE_BF16) {
-        lo = f32_to_bf16_bits(v[2 * e]);
-        hi = f32_to_bf16_bits(v[2 * e + 1]);
+        a[e] = f32_to_bf16_pair(v[2 * e], v[2 * e + 1]);
       } else {
-        lo = __builtin_bit_cast(uint16_t, static_cast<_Float16>(v[2 * e]));
-        hi = __builtin_bit_cast(uint16_t, static_cast<_Float16>(v[2 * e + 1]));
+        const uint32_t lo = __builtin_bit_cast(uint16_t, static_cast<_Float16>(v[2 * e]));
+        const uint32_t hi = __builtin_bit_cast(uint16_t, static_cast<_Float16>(v[2 * e + 1]));
+        a[e] = lo | (hi << 16);
       }
-      a[e] = lo | (hi << 16);
     }
     *reinterpret_cast<u32x4 *>(static_cast<uint16_t *>(p) + i) = a;
   }

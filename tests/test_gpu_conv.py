@@ -243,3 +243,19 @@ def test_fn_repeated_slot_id_with_mismatched_has_initial_state():
     assert bf16_close(y[:1], y0) and bf16_close(y[1:], y1)
     assert np.array_equal(np64(pool[3]), f0[0])
     assert torch.equal(pool[:3].cpu(), pool0[:3])
+
+
+@pytest.mark.parametrize("t", [1, 7, 8, 9, 40, 511, 512, 513, 1023, 1024, 1025])
+def test_short_inputs_give_the_bits_of_a_long_one(t):
+    """8-, 16- and 32-token tiles (t tokens alone) against the long tiles (the same tokens, history and pool row
+    packed ahead of 16,000 others); the sequence cut by tile ends at every remainder."""
+    gen = torch.Generator().manual_seed(t)
+    c = 8192
+    x = torch.randn(t + 16000, c, generator=gen).bfloat16().to(DEV)
+    w = (torch.randn(c, 4, generator=gen) * 0.5).bfloat16().to(DEV)
+    pools = [torch.randn(3, c, 4, generator=torch.Generator().manual_seed(1)).bfloat16().to(DEV) for _ in range(2)]
+    y = causal_conv1d_fn(x[:t], w, None, "silu", cu_seqlens=torch.tensor([0, t // 3, t], dtype=torch.int32, device=DEV),
+                         conv_states=pools[0], cache_indices=torch.tensor([2, 0], device=DEV))
+    ref = causal_conv1d_fn(x, w, None, "silu", conv_states=pools[1], cache_indices=torch.tensor([2, 0, -1], device=DEV),
+                           cu_seqlens=torch.tensor([0, t // 3, t, t + 16000], dtype=torch.int32, device=DEV))
+    assert torch.equal(y, ref[:t]) and torch.equal(pools[0], pools[1])
