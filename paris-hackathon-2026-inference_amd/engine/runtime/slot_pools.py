@@ -67,9 +67,10 @@ class GDNSlotPools:
             if r.device != self.device or c.device != self.device:
                 raise ValueError(f"layer {i}: pools on different devices")
         self.max_batch = int(max_batch or self.num_slots)
-        self._slots = torch.full((self.max_batch,), GDN_PAD_SLOT, dtype=torch.int64, device=self.device)
+        # the rows' slots, and the slots they start from (read_slots)
+        self._slots, self._read = torch.full((2, self.max_batch), GDN_PAD_SLOT, dtype=torch.int64,
+                                             device=self.device).unbind()
         self._has_state = torch.zeros(self.max_batch, dtype=torch.bool, device=self.device)
-        self._read = torch.full((self.max_batch,), GDN_PAD_SLOT, dtype=torch.int64, device=self.device)
         self.batch_size = 0
         self.decode = False
         self.verify_tokens = 0
@@ -115,9 +116,10 @@ class GDNSlotPools:
         ok = (ids >= 0) & (ids < self.num_slots)
         if b > 1:
             earlier = torch.tril(ids.unsqueeze(0) == ids.unsqueeze(1), diagonal=-1).any(dim=1)
-            ok &= ~earlier
-        self._slots[:b].copy_(torch.where(ok, ids, torch.full_like(ids, GDN_PAD_SLOT)))
-        self._slots[b:].fill_(GDN_PAD_SLOT)
+            ok = ok > earlier
+        self._slots[:b].copy_(torch.where(ok, ids, GDN_PAD_SLOT))
+        if b < self.max_batch:
+            self._slots[b:].fill_(GDN_PAD_SLOT)
         self._has_state.fill_(not is_prefill)
         if is_prefill:
             self._read.fill_(GDN_PAD_SLOT)
