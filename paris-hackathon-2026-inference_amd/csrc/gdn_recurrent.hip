@@ -340,7 +340,7 @@ __global__ __launch_bounds__(NT) void recurrent_kernel(RecArgs a) {
 // two or more waves of a SIMD together about every 5).  Measured, fp32, 32
 // v-heads of 128 x 128, from graphs, against recurrent_kernel: T = 256 at
 // B = 1 / 4 / 8 55.7 / 98.2 / 171.9 against 598 / 624 / 648 us; T = 1024 at
-// B = 1 208 against 2380.
+// B = 1, eager calls, 193 against 2380.
 constexpr int TOK_NT = 256;
 
 // Sum over the LPC (8 or 16) lanes that share a column, in every lane.
@@ -351,6 +351,18 @@ __device__ __forceinline__ float col_sum(float x) {
   x += dpp_mov<0x141>(x);                           // row_half_mirror
   if constexpr (LPC == 16) x += dpp_mov<0x140>(x);  // row_mirror
   return x;
+}
+
+// 1 / sqrt(x), x > 0, rounded once: the hardware's value (off by up to 1 ulp,
+// the same factor on a whole q or k row) and one Newton step whose residual is
+// exact to fp32.  Once per row and block; fp32 outputs against 64 bits, 1 x 1024
+// / 4 x 100 / 8 x 128 tokens: 1.000e-7 / 1.025e-7 / 1.023e-7 without it, 0.978e-7
+// / 1.005e-7 / 1.001e-7 with it (recurrent_kernel 0.994e-7 / 1.001e-7 / 0.998e-7),
+// for 190 -> 193 us at 1 x 1024.
+__device__ __forceinline__ float rsqrt_once(float x) {
+  const float r = rsqrtf(x), t = x * r;
+  const float e = __builtin_fmaf(-__builtin_fmaf(x, r, -t), r, __builtin_fmaf(-t, r, 1.f));  // 1 - x r^2
+  return x < __builtin_inff() ? __builtin_fmaf(0.5f * r, e, r) : r;
 }
 
 // ES: bytes of a q/k/v element (2 or 4); KD: k head dim; LPC, CPL: lanes per
@@ -458,8 +470,8 @@ __global__ __launch_bounds__(TOK_NT) void recurrent_tokens_kernel(RecArgs a) {
       sqq = row16_sum(sqq);
       skk = row16_sum(skk);
       sqk = row16_sum(sqk);
-      const float rq = (a.l2norm ? rsqrtf(sqq + 1e-6f) : 1.f) * a.scale;
-      const float rk = a.l2norm ? rsqrtf(skk + 1e-6f) : 1.f;
+      const float rq = (a.l2norm ? rsqrt_once(sqq + 1e-6f) : 1.f) * a.scale;
+      const float rk = a.l2norm ? rsqrt_once(skk + 1e-6f) : 1.f;
 #pragma unroll
       for (int e = 0; e < PER; e += 4) {
         *reinterpret_cast<f32x4 *>(&qt[t][l16 * PER + e]) = f32x4{qf[e], qf[e + 1], qf[e + 2], qf[e + 3]} * rq;
