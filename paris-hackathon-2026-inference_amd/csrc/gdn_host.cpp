@@ -23,6 +23,7 @@
 #include <limits>
 
 #include "gdn_capi.h"
+#include "gdn_gate_proj.h"
 
 namespace {
 
@@ -39,6 +40,7 @@ struct Entries {
   decltype(&gdn_out_proj_workspace_bytes) out_proj_workspace;
   decltype(&gdn_out_proj_decode) out_proj;
   decltype(&causal_conv1d_fwd) conv;
+  decltype(&gdn_gate_proj) gate_proj;
 } fn;
 
 using at::Tensor;
@@ -383,6 +385,38 @@ PyObject *out_proj(PyObject *, PyObject *const *a, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// gate_proj(hidden, w_b, w_a): hidden [..., K] contiguous bf16; (b, a), each [..., n]
+PyObject *gate_proj(PyObject *, PyObject *const *a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  bool ok = true;
+  if (n != 3) return none();
+  const Tensor *x = tensor(a[0], ok), *wb = tensor(a[1], ok), *wa = tensor(a[2], ok);
+  if (!ok || !x || !wb || !wa || !same_device(*x, {wb, wa})) return none();
+  if (x->scalar_type() != at::kBFloat16 || x->dim() < 2 || x->numel() == 0 || !x->is_contiguous() ||
+      reinterpret_cast<uintptr_t>(x->data_ptr()) % 16)
+    return none();
+  const int64_t k = x->size(-1), m = x->numel() / k;
+  if (!bf16_matrix(wb, k) || !bf16_matrix(wa, k) || !fits32(m)) return none();
+  const int64_t cols = wb->size(0);
+  if (wa->size(0) != cols || (cols != 16 && cols != 32) || (k != 1024 && k != 2048)) return none();
+  Tensor out[2];
+  int st;
+  {
+    NoGil unlocked;
+    auto sizes = x->sizes().vec();
+    sizes.back() = cols;
+    for (Tensor &t : out) t = empty(sizes, *x);
+    st = fn.gate_proj(x->data_ptr(), wb->data_ptr(), wa->data_ptr(), m, k, cols, out[0].data_ptr(), out[1].data_ptr(),
+                      stream_of(*x));
+  }
+  if (st) return failed("gdn_gate_proj", st);
+  PyObject *r = PyTuple_New(2);
+  if (!r) return nullptr;
+  for (int i = 0; i < 2; ++i) PyTuple_SET_ITEM(r, i, THPVariable_Wrap(out[i]));
+  return r;
+  END_HANDLE_TH_ERRORS
+}
+
 // conv(x, weight, bias, silu, pool, idx, read_idx, cu): x [tokens, C], or [B, C, T] with the channels
 // contiguous, in the weight's dtype; read_idx None: the history comes through idx.  Returns y laid out as x.
 PyObject *conv(PyObject *, PyObject *const *a, Py_ssize_t n) {
@@ -507,7 +541,7 @@ PyObject *bind(PyObject *, PyObject *const *a, Py_ssize_t n) {
 #define GDN_METHOD(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(name)), METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {GDN_METHOD(bind),    GDN_METHOD(recurrent), GDN_METHOD(chunk),
                          GDN_METHOD(rms_norm), GDN_METHOD(in_proj),   GDN_METHOD(out_proj),
-                         GDN_METHOD(conv),     GDN_METHOD(core_decode), {nullptr, nullptr, 0, nullptr}};
+                         GDN_METHOD(conv),     GDN_METHOD(core_decode), GDN_METHOD(gate_proj), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_gdn_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace

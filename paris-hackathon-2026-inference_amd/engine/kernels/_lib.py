@@ -129,7 +129,8 @@ HOST_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "_gdn_host.
 # the entry points that the host extension calls, in its order (csrc/gdn_host.cpp: Entries)
 HOST_ENTRIES = ("gdn_last_error_string", "gdn_recurrent_fwd", "gdn_recurrent_fwd_gated", "gdn_chunk_fwd",
                 "gdn_chunk_fwd_gated", "gdn_chunk_workspace_bytes", "gdn_rmsnorm_gated_fwd", "gdn_in_proj_decode",
-                "gdn_out_proj_workspace_bytes", "gdn_out_proj_decode", "causal_conv1d_fwd")
+                "gdn_out_proj_workspace_bytes", "gdn_out_proj_decode", "causal_conv1d_fwd",
+                "gdn_gate_proj")
 
 
 def load(path: str = LIB_PATH) -> ctypes.CDLL:

@@ -131,6 +131,22 @@ def _fused_decode(self, hidden_states: torch.Tensor, conv_state: torch.Tensor,
                               slots, self.activation)
 
 
+def _gate_projections(self, hidden_states: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
+    """``(in_proj_b(x), in_proj_a(x))``: one kernel for both where they are
+    plain bias-free bf16 ``nn.Linear`` modules without hooks and no gradient
+    is recorded (csrc/gdn_gate_proj.hip), else the modules."""
+    lb, la = self.in_proj_b, self.in_proj_a
+    if type(lb) is type(la) is torch.nn.Linear and not (
+            lb._forward_hooks or lb._forward_pre_hooks or la._forward_hooks or la._forward_pre_hooks):
+        (wb, bias_b), (wa, bias_a) = _weight_bias(lb), _weight_bias(la)
+        if bias_b is None and bias_a is None and not torch.is_autocast_enabled("cuda") and not (
+                torch.is_grad_enabled() and (hidden_states.requires_grad or wb.requires_grad or wa.requires_grad)):
+            done = _lib.host().gate_proj(hidden_states, wb, wa)
+            if done is not None:
+                return done
+    return lb(hidden_states), la(hidden_states)
+
+
 def _out_proj_fits(self, out: torch.Tensor) -> bool:
     """Whether ``out_proj`` over these rows can take :func:`gdn_out_proj_decode`:
     one token per row, at most OUT_PROJ_MAX_M rows, a plain bias-free bf16
@@ -173,8 +189,7 @@ def gated_delta_net_forward(self, hidden_states: torch.Tensor, cache_params=None
     else:
         mixed_qkv = self.in_proj_qkv(hidden_states).transpose(1, 2)
         z = self.in_proj_z(hidden_states)
-        b = self.in_proj_b(hidden_states)
-        a = self.in_proj_a(hidden_states)
+        b, a = _gate_projections(self, hidden_states)
         conv_w = self.conv1d.weight.squeeze(1)
         if decode_step:
             mixed_qkv = causal_conv1d_update(mixed_qkv, layer.conv_states[0], conv_w, self.conv1d.bias,
@@ -267,8 +282,7 @@ def _forward_on_pools(self, hidden_states: torch.Tensor, pools, attention_mask: 
     else:
         mixed_qkv = self.in_proj_qkv(hidden_states).transpose(1, 2)  # [B, conv_dim, L]
         z = self.in_proj_z(hidden_states)
-        b = self.in_proj_b(hidden_states)
-        a = self.in_proj_a(hidden_states)
+        b, a = _gate_projections(self, hidden_states)
         conv_w = self.conv1d.weight.squeeze(1)
         if step:
             mixed_qkv = causal_conv1d_update(mixed_qkv, conv_pool, conv_w, self.conv1d.bias, self.activation,
