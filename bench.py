@@ -308,8 +308,7 @@ def bench_prefill_b16(torch, reps=100, repeat_qk=False):
     """The reference's own profiled prefill shape (its profile of fla's chunk
     kernel: 1.659 ms per layer on H200): a dense batch of 16 sequences of 1038
     tokens (17 chunks each), q/k at 16 heads (with repeat_qk: repeated to the
-    32 v-heads, as HF passes them), v at 32, zero h0, final states out; the
-    batch is scanned by the persistent scan."""
+    32 v-heads, as HF passes them), v at 32, zero h0, final states out."""
     from engine import configs
     from engine.kernels import chunk_gated_delta_rule
 

@@ -16,8 +16,8 @@ the kernel prologues (``*_from_projections``), q/k passed at their 16 heads
 (native GQA), and the norm as one HIP pass (:func:`rms_norm_gated`).  A
 one-token decode step runs the four input projections and the conv update
 as one HIP kernel (:func:`engine.kernels.in_proj.gdn_in_proj_decode`);
-otherwise the projections are torch matmuls (hipBLASLt) and the conv runs
-the HIP ``causal_conv1d`` kernels on their output in place.  The cache calls
+otherwise qkv, z (and out) are torch matmuls (hipBLASLt), b and a one kernel
+where they have its form (:func:`_gate_projections`), and the conv runs the HIP ``causal_conv1d`` kernels on their output in place.  The cache calls
 are HF's own, in HF's order, so the layer works with the transformers cache
 unchanged.  With an engine
 slot-pool cache (``cache_params.gdn_slot_pools``, see
