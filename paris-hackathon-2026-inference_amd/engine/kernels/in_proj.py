@@ -11,8 +11,9 @@ projection goes through the conv window update in registers, so it is never
 written out before the conv.  :func:`gdn_out_proj_decode` runs ``out_proj``
 (:428, called at :540) for decode rows with K split over 256 workgroups (the
 2048 output columns alone would occupy 32).  Prefill keeps the library GEMMs
-(hipBLASLt via ``torch.nn.functional.linear``): there the projections are
-compute-bound and the conv kernels read their output in place.
+(hipBLASLt via ``torch.nn.functional.linear``) for qkv, z and out: there they
+are compute-bound and the conv kernels read their output in place; b and a, 32
+columns each, run in one kernel (csrc/gdn_gate_proj.hip).
 """
 from __future__ import annotations
 
