@@ -131,13 +131,32 @@ def _fused_decode(self, hidden_states: torch.Tensor, conv_state: torch.Tensor,
                               slots, self.activation)
 
 
+_LINEAR_FORWARD = torch.nn.Linear.forward
+
+
+def _only_its_product(lin) -> bool:
+    """Whether calling ``lin`` is ``nn.Linear``'s product and nothing else: no
+    subclass, no ``forward`` set on the instance (as adapter and offload tools
+    attach) or in the class's place, no hooks of its own."""
+    return (type(lin) is torch.nn.Linear and "forward" not in lin.__dict__
+            and torch.nn.Linear.forward is _LINEAR_FORWARD
+            and not (lin._forward_hooks or lin._forward_pre_hooks or lin._backward_hooks or lin._backward_pre_hooks))
+
+
+def _modules_observed() -> bool:
+    """Whether something outside a module sees its call: hooks registered for
+    all modules, or a torch function or dispatch mode."""
+    return bool(torch.nn.modules.module._has_any_global_hook() or torch._C._len_torch_function_stack()
+                or torch._C._len_torch_dispatch_stack())
+
+
 def _gate_projections(self, hidden_states: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
     """``(in_proj_b(x), in_proj_a(x))``: one kernel for both where they are
-    plain bias-free bf16 ``nn.Linear`` modules without hooks and no gradient
-    is recorded (csrc/gdn_gate_proj.hip), else the modules."""
+    bias-free bf16 ``nn.Linear`` modules whose call is their product alone
+    (:func:`_only_its_product`, :func:`_modules_observed`) and no gradient is
+    recorded (csrc/gdn_gate_proj.hip), else the modules."""
     lb, la = self.in_proj_b, self.in_proj_a
-    if type(lb) is type(la) is torch.nn.Linear and not (
-            lb._forward_hooks or lb._forward_pre_hooks or la._forward_hooks or la._forward_pre_hooks):
+    if _only_its_product(lb) and _only_its_product(la) and not _modules_observed():
         (wb, bias_b), (wa, bias_a) = _weight_bias(lb), _weight_bias(la)
         if bias_b is None and bias_a is None and not torch.is_autocast_enabled("cuda") and not (
                 torch.is_grad_enabled() and (hidden_states.requires_grad or wb.requires_grad or wa.requires_grad)):
