@@ -88,14 +88,16 @@ def rms_norm_gated(x: torch.Tensor, z: torch.Tensor, weight: torch.Tensor, eps: 
 def _weight_bias(lin) -> tuple:
     """A projection's weight and bias, from its parameter table where they
     are plain parameters (an ``nn.Module`` attribute costs the interpreter a
-    microsecond)."""
+    microsecond), else its attributes."""
+    if not isinstance(lin, torch.nn.Module):
+        return lin.weight, lin.bias
     table = lin._parameters
     w = table.get("weight")
     return (lin.weight if w is None else w), (table["bias"] if "bias" in table else lin.bias)
 
 
 def _projections(self) -> list:
-    mods = self._modules
+    mods = self._modules if isinstance(self, torch.nn.Module) else {}
     return [mods[n] if n in mods else getattr(self, n)
             for n in ("in_proj_qkv", "in_proj_z", "in_proj_b", "in_proj_a", "conv1d")]
 
@@ -260,6 +262,8 @@ def _native_core(self, qkv: torch.Tensor, z: torch.Tensor, b: torch.Tensor, a: t
     recurrence on the pools and the gated norm (the kernels of the general way
     below, in its order), ``[B, 1, Hv*V]``; None where its form is not the
     regular one."""
+    if not isinstance(self, torch.nn.Module):
+        return None
     params, norm = self._parameters, self._modules.get("norm")
     alog, dtb = params.get("A_log"), params.get("dt_bias")
     if alog is None or dtb is None or norm is None:

@@ -1,13 +1,14 @@
-"""Forms of the layer's modules that the fused forward accepts, on the CPU:
-which ones the two gate projections leave to the modules (no kernel runs
-here; the host extension is a stand-in that takes every call)."""
+"""Forms of the layer and its modules that the fused forward accepts, on the CPU:
+bare objects with the same attributes, and which modules the two gate
+projections leave to their own calls (no kernel runs here; the host extension
+is a stand-in that takes every call)."""
 import types
 
 import pytest
 import torch
 import torch.utils._python_dispatch
 
-from engine.kernels import _lib
+from engine.kernels import _lib, gdn_layer
 from engine.kernels.gdn_layer import _gate_projections
 
 TAKEN = ("b from the kernel", "a from the kernel")
@@ -100,3 +101,31 @@ def test_gate_projections_under_a_mode_run_as_modules(takes_all, mode):
     with mode():
         check(lay, False)
     check(lay, True)
+
+
+def plain_objects(kind, k=1024):
+    """A layer's projections as bare objects that hold a weight and a bias, in a bare layer object or a module."""
+    def lin(*shape):
+        return types.SimpleNamespace(weight=torch.zeros(*shape, dtype=torch.bfloat16), bias=None)
+
+    lay = types.SimpleNamespace() if kind == "layer" else torch.nn.Module()
+    lay.in_proj_qkv, lay.in_proj_z, lay.in_proj_b, lay.in_proj_a = lin(1024, k), lin(512, k), lin(4, k), lin(4, k)
+    lay.conv1d = lin(1024, 1, 4)
+    lay.activation = "silu"
+    return lay
+
+
+@pytest.mark.parametrize("kind", ["layer", "projections"])
+def test_layers_and_projections_need_not_be_modules(monkeypatch, kind):
+    lay = plain_objects(kind)
+    windows = torch.zeros(3, 1024, 4, dtype=torch.bfloat16)
+    assert gdn_layer._fused_decode_fits(lay, torch.zeros(2, 1, 1024).bfloat16(), windows)
+    assert not gdn_layer._fused_decode_fits(lay, torch.zeros(2, 1, 512).bfloat16(), windows)
+    seen = []
+    monkeypatch.setattr(gdn_layer, "gdn_in_proj_decode", lambda *a: seen.append(a))
+    gdn_layer._fused_decode(lay, "x", windows, "slots")
+    names = ("in_proj_qkv", "in_proj_z", "in_proj_b", "in_proj_a")
+    assert all(a is getattr(lay, n).weight for a, n in zip(seen[0][1:5], names))
+    assert seen[0][5] is lay.conv1d.weight and seen[0][6] is None
+    # between the projections such a layer goes the general way
+    assert gdn_layer._native_core(types.SimpleNamespace(), *(None,) * 6) is None
