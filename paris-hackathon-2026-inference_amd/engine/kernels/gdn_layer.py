@@ -296,6 +296,7 @@ def _forward_on_pools(self, hidden_states: torch.Tensor, pools, attention_mask: 
     # fused decode input side (which moves the window on) or the chunk kernels
     # (which keep no snapshots)
     step = pools.decode and seq_len == 1 and not verify
+    read_slots = None if step else pools.read_slots()
     if step and _fused_decode_fits(self, hidden_states, conv_pool):
         projected = _fused_decode(self, hidden_states, conv_pool, slots)
         out = _native_core(self, *projected, slots, rec_pool)
@@ -314,7 +315,7 @@ def _forward_on_pools(self, hidden_states: torch.Tensor, pools, attention_mask: 
             if verify:
                 pools.record_conv(self.layer_idx, mixed_qkv)
             mixed_qkv = _conv1d_fn(mixed_qkv, conv_w, self.conv1d.bias, self.activation, conv_states=conv_pool,
-                                   cache_indices=slots, read_indices=pools.read_slots())
+                                   cache_indices=slots, read_indices=read_slots)
         mixed_qkv = mixed_qkv.transpose(1, 2)
     query, key, value = torch.split(mixed_qkv, [self.key_dim, self.key_dim, self.value_dim], dim=-1)
     query = query.reshape(batch_size, seq_len, -1, self.head_k_dim)
@@ -327,7 +328,7 @@ def _forward_on_pools(self, hidden_states: torch.Tensor, pools, attention_mask: 
             snapshots=pools.snapshots(self.layer_idx) if verify else None)
     else:
         core, _ = _from_projections(query, key, value, a, b, self.A_log, self.dt_bias, rec_pool, False, True, None,
-                                    None, slots, True, read_indices=pools.read_slots())
+                                    None, slots, True, read_indices=read_slots)
 
     z = z.reshape(batch_size, seq_len, -1, self.head_v_dim)
     out = rms_norm_gated(core, z, self.norm.weight, self.norm.variance_epsilon)

@@ -67,9 +67,8 @@ class GDNSlotPools:
             if r.device != self.device or c.device != self.device:
                 raise ValueError(f"layer {i}: pools on different devices")
         self.max_batch = int(max_batch or self.num_slots)
-        # the rows' slots, and the slots they start from (read_slots)
-        self._slots, self._read = torch.full((2, self.max_batch), GDN_PAD_SLOT, dtype=torch.int64,
-                                             device=self.device).unbind()
+        self._slots = torch.full((self.max_batch,), GDN_PAD_SLOT, dtype=torch.int64, device=self.device)
+        self._pad = torch.full((), GDN_PAD_SLOT, dtype=torch.int64, device=self.device)
         self._has_state = torch.zeros(self.max_batch, dtype=torch.bool, device=self.device)
         self.batch_size = 0
         self.decode = False
@@ -121,10 +120,6 @@ class GDNSlotPools:
         if b < self.max_batch:
             self._slots[b:].fill_(GDN_PAD_SLOT)
         self._has_state.fill_(not is_prefill)
-        if is_prefill:
-            self._read.fill_(GDN_PAD_SLOT)
-        else:
-            self._read.copy_(self._slots)
         self.batch_size = b
         self.decode = not is_prefill
         if verify_tokens:
@@ -136,14 +131,17 @@ class GDNSlotPools:
         return self._slots[: self.batch_size]
 
     def has_state(self) -> torch.Tensor:
-        """Per row: continue from the slot's state (decode) or start from zero (prefill)."""
+        """Per row: continue from the slot's state (decode) or start from zero
+        (prefill).  A view of a persistent buffer: rows marked in it after
+        :meth:`bind` start as marked in every later conv and chunk prefill of
+        the bound batch (replays of a captured one included)."""
         return self._has_state[: self.batch_size]
 
     def read_slots(self) -> torch.Tensor:
-        """Slot ids the bound batch's rows start from (a view of a persistent
-        buffer): the rows' own slots in a decode step, ``GDN_PAD_SLOT`` (a zero
-        state and window) in a prefill."""
-        return self._read[: self.batch_size]
+        """Slot ids the bound batch's rows start from, by :meth:`has_state`
+        as it is on the device when this runs: a row's own slot, or
+        ``GDN_PAD_SLOT`` (a zero state and window)."""
+        return torch.where(self.has_state(), self.slots(), self._pad)
 
     def layer(self, layer_idx: int) -> Tuple[torch.Tensor, torch.Tensor]:
         """(conv pool, recurrent pool) of a GDN layer."""
