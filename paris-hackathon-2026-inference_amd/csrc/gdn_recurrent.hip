@@ -18,6 +18,8 @@
 //
 // Semantics: transformers modeling_qwen3_5_moe.py:331-381 (the torch
 // recurrence the reference imports at engine/runtime/cuda_graphs.py:126-135).
+#include <algorithm>
+
 #include "gdn_common.h"
 
 namespace gdn {
@@ -654,13 +656,31 @@ namespace {
 
 // Tokens per sequence (their average, with cu_seqlens) from which a call
 // without snapshots takes recurrent_tokens_kernel.  Its token steps are much
-// cheaper, its state accesses less contiguous (16 or 32 columns of a row per
-// workgroup).  Measured from graphs, fp32, 32 v-heads of 128 x 128, this kernel
-// against recurrent_kernel: T = 4 at B = 1 / 4 / 8 7 / 10.6 / 15-17 against
-// 12.2 / 13.5 / 15.8 us; T = 8 at B = 8 / 16 / 64 17.4 / 31-34 / 108-125
-// against 27.1 / 32.3 / 97.7; T = 16 at B = 16 / 64 38.6 / 129-146 against
-// 54.3 / 156.
-inline int64_t tokens_min(int64_t pairs) { return pairs <= 128 ? 4 : pairs <= 256 ? 8 : 16; }
+// cheaper, its state accesses less contiguous (16 to 64 columns of a row per
+// workgroup), so the line rises with the state a call moves.  Measured from
+// graphs, this kernel against recurrent_kernel, us:
+//   128 x 128, 32 v-heads, fp32: T = 4 at B = 1 / 4 / 8 7 / 10.6 / 15-17 against
+//   12.2 / 13.5 / 15.8; T = 8 at B = 8 / 16 / 64 17.4 / 31-34 / 108-125 against
+//   27.1 / 32.3 / 97.7; T = 16 at B = 16 / 64 38.6 / 129-146 against 54.3 / 156;
+//   256 x 256, bf16: T = 4 at 32 / 64 / 128 pairs 0.76 / 1.20 / 1.28 of
+//   recurrent_kernel's time, T = 6 at 64 / 128 0.97 / 1.08, T = 8 0.82 / 0.94
+//   (256 x 128 at 96 / 128 pairs: T = 4 0.89 / 1.20, T = 6 0.68 / 0.95);
+//   128 x 256, bf16: T = 4 at 64 / 96 pairs 0.85 / 1.13, T = 6 at 96 0.90; T = 8 at
+//   160 / 256 pairs 1.11 / 1.09, T = 12 0.89 / 0.91;
+//   64 x 64, bf16: T = 16 at 1,024 / 2,048 pairs 0.81 / 1.14, T = 24 0.63 / 0.92 (fp32,
+//   T = 16: 0.64 / 0.89).
+inline int64_t tokens_min(int64_t pairs, int K, int V, int64_t es) {
+  const int64_t cols = pairs * V;
+  const int64_t few = pairs <= 128 ? 4 : pairs <= 256 ? 8 : 16;
+  int64_t wide = 0;
+  if (K == 256)
+    wide = cols > 96 * 128 ? 8 : 0;
+  else if (K == 128)
+    wide = cols > 256 * 128 ? 12 : cols > 128 * 128 ? 6 : 0;
+  else
+    wide = es == 2 && cols > 512 * 128 ? 24 : 0;
+  return std::max(few, wide);
+}
 
 // State columns (pairs x V) from which more rows per lane pay: below
 // REC_TOKENS_MID_COLS a wave per SIMD is all there is and the shortest step
@@ -731,7 +751,8 @@ int recurrent_fwd(const void *q, const void *k, const void *v, int qkv_dtype,
   const int64_t es = static_cast<int64_t>(dtype_size(qkv_dtype));
   const bool aligned = (reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k)) % 16 == 0 &&
                        (q_stride_t * es) % 16 == 0 && (k_stride_t * es) % 16 == 0;
-  if (!snapshots && aligned && a.total >= tokens_min(static_cast<int64_t>(n_seqs) * Hv) * n_seqs && n_blocks * 2 <= 0x7fffffff) {
+  if (!snapshots && aligned && n_blocks * 2 <= 0x7fffffff &&
+      a.total >= tokens_min(static_cast<int64_t>(n_seqs) * Hv, K, V, es) * n_seqs) {
     if (es == 2)
       K == 64 ? launch_tokens<2, 64>(a, st) : K == 128 ? launch_tokens<2, 128>(a, st) : launch_tokens<2, 256>(a, st);
     else
