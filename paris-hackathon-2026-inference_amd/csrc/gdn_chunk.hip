@@ -2072,8 +2072,6 @@ int chunk_fwd(const void *q, const void *k, const void *v, int qkv_dtype,
   const int64_t longest = cu_seqlens ? (total + CK - 1) / CK : (T + CK - 1) / CK;  // chunks, or their bound
   const bool local = pairs >= LOC_MIN_PAIRS || longest == 1 || (longest == 2 && pairs >= LOC_SHORT2_PAIRS);
   const bool multi = nc > SEG_ONE;  // several segments
-  const int64_t seg = multi ? SEG_CHUNKS : nc;
-  const WsLayout l = ws_layout(n_seqs, seg, Hv, multi);
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (local) {  // one workgroup per (sequence, v-head); no workspace
     if (pairs > 0x7fffffff) return fail(GDN_ERR_INVALID_ARGUMENT, "%s: grid too large", name);
@@ -2088,18 +2086,31 @@ int chunk_fwd(const void *q, const void *k, const void *v, int qkv_dtype,
       hipLaunchKernelGGL((chunk_local_kernel<false>), grid, dim3(64 * LOC_WAVES), 0, s, a);
     return check_launch(name);
   }
-  if (!workspace || workspace_bytes < l.total)
-    return fail(GDN_ERR_WORKSPACE, "%s: workspace %zu bytes < %zu needed", name, workspace_bytes, l.total);
-  if (reinterpret_cast<uintptr_t>(workspace) % 256)
-    return fail(GDN_ERR_WORKSPACE, "%s: workspace must be 256-byte aligned", name);
-  if (nc > 65535) return fail(GDN_ERR_INVALID_ARGUMENT, "%s: %lld chunks exceed one launch", name, (long long)nc);
   // Several sequences of one length, several segments: a segment takes the
   // same window of chunks of every sequence, so that all of them are scanned
   // at once.  (With cu_seqlens the lengths are on the device: sequence after
   // sequence, and a segment holds few of them.)
   const int64_t chunks = (static_cast<int64_t>(T) + CK - 1) / CK;  // per sequence (dense)
-  const int win = multi && !cu_seqlens && n_seqs > 1 && n_seqs <= SEG_CHUNKS ? SEG_CHUNKS / n_seqs : 0;
-  const int64_t nseg = win ? (chunks + win - 1) / win : seg > 0 ? (nc + seg - 1) / seg : 0;
+  int win = multi && !cu_seqlens && n_seqs > 1 && n_seqs <= SEG_CHUNKS ? SEG_CHUNKS / n_seqs : 0;
+  auto windows = [&](int w) { return (chunks + w - 1) / w; };
+  // Sequence counts that leave over an eighth of the 64 slots idle (33 of them:
+  // 31) take up to SEG_ONE, for which gdn_chunk_workspace_bytes has room,
+  // where that saves a segment.  Hv = 4, 33 x 300 / 600 / 1300 tokens in windows
+  // of 1 chunk 129 / 253 / 549 us, of 2 chunks 92 / 162 / 354 (sequence after
+  // sequence 107 / 220 / 477).  Not always: more slots leave the Infinity Cache
+  // sooner (Hv = 32, B = 4 x T = 4096 in 80 slots 359 us, in 64 321).
+  if (win && 8 * win * n_seqs < 7 * SEG_CHUNKS) {
+    const int wide = SEG_ONE / n_seqs;
+    if (windows(wide) < windows(win) && workspace_bytes >= ws_layout(n_seqs, wide * n_seqs, Hv, true).total) win = wide;
+  }
+  const int64_t seg = !multi ? nc : win ? std::max<int64_t>(SEG_CHUNKS, win * n_seqs) : SEG_CHUNKS;
+  const WsLayout l = ws_layout(n_seqs, seg, Hv, multi);
+  if (!workspace || workspace_bytes < l.total)
+    return fail(GDN_ERR_WORKSPACE, "%s: workspace %zu bytes < %zu needed", name, workspace_bytes, l.total);
+  if (reinterpret_cast<uintptr_t>(workspace) % 256)
+    return fail(GDN_ERR_WORKSPACE, "%s: workspace must be 256-byte aligned", name);
+  if (nc > 65535) return fail(GDN_ERR_INVALID_ARGUMENT, "%s: %lld chunks exceed one launch", name, (long long)nc);
+  const int64_t nseg = win ? windows(win) : seg > 0 ? (nc + seg - 1) / seg : 0;
   // (sequence, v-head) pairs whose chains run at the same time
   const int64_t active = multi && !win ? Hv : pairs;
   char *ws = static_cast<char *>(workspace);

@@ -591,6 +591,13 @@ def test_column_scan_matches_the_oracle(n, hv, t):
     assert torch.equal(o2, o) and torch.equal(s2, s)
 
 
+# windows of several sequences with at most 32 pairs (16 columns per workgroup), and sequence counts
+# whose windows take more than 64 slots: 33 x 2, 39 x 2 and 24 x 3 chunks
+@pytest.mark.parametrize("n,hv,t", [(2, 4, 2700), (8, 4, 700), (2, 16, 2650), (33, 4, 300), (39, 2, 193), (24, 4, 300)])
+def test_windows_match_the_oracle(n, hv, t):
+    test_column_scan_matches_the_oracle(n, hv, t)
+
+
 @pytest.mark.parametrize("lens,hv", [([200, 0, 64, 65, 1, 0, 130, 17, 63, 128], 4), ([100] * 17, 4),
                                      ([900, 0, 3000, 64, 2000], 8), ([5200], 2)])
 def test_column_scan_packed_on_a_slot_pool(lens, hv):

@@ -1,12 +1,15 @@
-"""Which kernel a call takes, at the lines of the dispatch rules (both sides
+"""Which kernels a call takes, at the lines of the dispatch rules (both sides
 of a line are right; the rules say which one is faster).  A recurrence with
 snapshots always runs the per-token kernel, so a call without them that takes
 that kernel too gives its bits, and one that takes the token-block kernel
-gives others (sums in another order)."""
+gives others (sums in another order).  A chunk prefill's segments are counted
+as the launches that it records into a graph."""
+import ctypes
+
 import pytest
 import torch
 
-from engine.kernels import fused_recurrent_gated_delta_rule
+from engine.kernels import _lib, chunk_gated_delta_rule, fused_recurrent_gated_delta_rule
 
 pytestmark = [pytest.mark.gpu,
               pytest.mark.skipif(not torch.cuda.is_available(), reason="needs an MI355X")]
@@ -42,3 +45,60 @@ def test_short_recurrences_take_the_faster_kernel(kd, vd, dt, n, hv, t, blocks):
     one, other = last(), last(snapshots=torch.empty(n, t, hv, kd, vd, device=DEV))
     assert torch.equal(one, other) == (not blocks)
     assert (one - other).norm() <= 1e-5 * other.norm()
+
+
+def kernels_of(call):
+    """The number of nodes that ``call`` records into a graph (its launches)."""
+    call()
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        call()
+    with open("/proc/self/maps") as f:  # the runtime that torch loaded
+        hip = ctypes.CDLL(next(line.split()[-1] for line in f if "libamdhip64.so" in line))
+    count = ctypes.c_size_t()
+    assert hip.hipGraphGetNodes(ctypes.c_void_p(graph.raw_cuda_graph()), None, ctypes.byref(count)) == 0
+    return count.value
+
+
+def chunk_args(n, t, hv):
+    gen = torch.Generator(device=DEV).manual_seed(n + t)
+    q, k, v = (torch.randn(n, t, h, 128, generator=gen, device=DEV).to(BF16) for h in (hv // 2, hv // 2, hv))
+    g, beta = -torch.rand(n, t, hv, generator=gen, device=DEV), torch.rand(n, t, hv, generator=gen, device=DEV)
+    return q, k, v, g, beta, torch.randn(n, hv, 128, 128, generator=gen, device=DEV)
+
+
+# sequences, v-heads, tokens, segments (a prep and a scan launch each): one up to 80 chunks in all; windows
+# in 64 slots, in 80 where those save a segment; one sequence
+@pytest.mark.parametrize("n,hv,t,segments", [
+    (10, 4, 512, 1), (10, 4, 513, 2), (4, 8, 1400, 2), (17, 4, 300, 2), (24, 4, 300, 2), (32, 4, 300, 3),
+    (33, 4, 300, 3), (33, 4, 1300, 11), (39, 4, 450, 4), (48, 2, 200, 4), (1, 4, 5120, 1), (1, 4, 5121, 2)])
+def test_segments_of_dense_batches(n, hv, t, segments):
+    q, k, v, g, beta, h0 = chunk_args(n, t, hv)
+    assert kernels_of(lambda: chunk_gated_delta_rule(q, k, v, g, beta, initial_state=h0, output_final_state=True,
+                                                     use_qk_l2norm_in_kernel=True)) == 2 * segments
+
+
+def test_a_workspace_of_64_chunks_still_serves():
+    """33 sequences in windows of two chunks use 66 slots where the workspace has them, one chunk where not."""
+    n, t, hv = 33, 300, 4
+    q, k, v, g, beta, h0 = chunk_args(n, t, hv)
+    lib, out = _lib.load(), []
+    full = lib.gdn_chunk_workspace_bytes(n, n * t, hv, 128, 128)
+    slot = hv * (25 + 32) * 1024  # a chunk's operands: 25 blocks and U per v-head
+    ws = torch.empty(full, dtype=torch.uint8, device=DEV)
+
+    def call(bytes_):
+        o, s = torch.empty_like(v), torch.empty_like(h0)
+        st = lib.gdn_chunk_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), _lib.GDN_DTYPE[BF16], hv // 2 * 128, hv // 2 * 128,
+                               hv * 128, g.data_ptr(), beta.data_ptr(), 0, h0.data_ptr(), None, n, s.data_ptr(), None, n,
+                               o.data_ptr(), _lib.GDN_DTYPE[BF16], None, n, t, hv // 2, hv, 128, 128, 128 ** -0.5, 1,
+                               ws.data_ptr(), bytes_, _lib.stream_of(q))
+        out.append((o, s))
+        return st
+
+    assert call(full - 17 * slot) != 0  # 63 slots: refused
+    for bytes_, launches in ((full, 6), (full - 15 * slot, 10)):
+        assert kernels_of(lambda: call(bytes_)) == launches
+    (o, s), (o2, s2) = out[1], out[3]  # (out[2], out[4]: captured, not run)
+    assert torch.equal(o, o2) and torch.equal(s, s2)
