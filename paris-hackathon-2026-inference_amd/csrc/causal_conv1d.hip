@@ -25,7 +25,10 @@ constexpr int CONV_NT = 256;   // threads per workgroup
 // (short inputs are bound by a tile's serial walk: 100 / 333 / 512 tokens of
 // 8192 channels with tiles of 8 / 16 / 32 8.3 / 9.6 / 12.5, 9.0 / 11.0 / 13.1
 // and 9.9 / 11.3 / 14.0 us; 1,024 tokens with 16 / 32 12.8 / 15.1; a second round
-// costs more than it saves: 750 tokens with 8 14.7 against 12.4 with 16), 32 when
+// costs more than it saves: 750 tokens with 8 14.7 against 12.4 with 16; the same
+// at 256 to 12288 channels in bf16 and fp32, but that beyond 32 million bytes of x
+// the halo re-read costs more than 16 saves: fp32, 2048 channels, 3,600 / 4,000 /
+// 4,096 tokens with 16 / 32 16.7 / 17.2, 18.2 / 17.8 and 18.4 / 17.7 us), 32 when
 // a 64-token grid would leave CUs without a workgroup, else the longest of 64, 56 and 48
 // whose busiest CU streams the fewest tokens, ceil(workgroups / CUs) x tile:
 // a long tile halves the re-read 3-token halo against 32 and keeps more loads
@@ -34,6 +37,7 @@ constexpr int CONV_NT = 256;   // threads per workgroup
 // 13,794 tokens: 864 workgroups of 64 tokens, 3.4 per CU; 988 of 56)
 constexpr int TILE_SHORT = 32, TILE_LONG = 64;
 constexpr int CONV_CUS = 256;
+constexpr int64_t TILE16_BYTES = 32000000;
 
 template <typename T> struct Vec8;
 template <> struct Vec8<uint16_t> {
@@ -385,7 +389,7 @@ int launch_fwd(const ConvArgs &a, hipStream_t s) {
     };
     if (workgroups(8) <= CONV_CUS) {
       launch_tiles<T, SL, 8>(a, gx, s);
-    } else if (workgroups(16) <= CONV_CUS) {
+    } else if (workgroups(16) <= CONV_CUS && a.total * a.C * static_cast<int64_t>(sizeof(T)) <= TILE16_BYTES) {
       launch_tiles<T, SL, 16>(a, gx, s);
     } else if (workgroups(TILE_LONG) < CONV_CUS) {
       launch_tiles<T, SL, TILE_SHORT>(a, gx, s);

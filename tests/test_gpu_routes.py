@@ -2,14 +2,14 @@
 of a line are right; the rules say which one is faster).  A recurrence with
 snapshots always runs the per-token kernel, so a call without them that takes
 that kernel too gives its bits, and one that takes the token-block kernel
-gives others (sums in another order).  A chunk prefill's segments are counted
-as the launches that it records into a graph."""
+gives others (sums in another order).  Other routes are read off the launches that a
+call records into a graph."""
 import ctypes
 
 import pytest
 import torch
 
-from engine.kernels import _lib, chunk_gated_delta_rule, fused_recurrent_gated_delta_rule
+from engine.kernels import _lib, causal_conv1d_fn, chunk_gated_delta_rule, fused_recurrent_gated_delta_rule
 
 pytestmark = [pytest.mark.gpu,
               pytest.mark.skipif(not torch.cuda.is_available(), reason="needs an MI355X")]
@@ -47,8 +47,17 @@ def test_short_recurrences_take_the_faster_kernel(kd, vd, dt, n, hv, t, blocks):
     assert (one - other).norm() <= 1e-5 * other.norm()
 
 
-def kernels_of(call):
-    """The number of nodes that ``call`` records into a graph (its launches)."""
+class Dim3(ctypes.Structure):
+    _fields_ = [(n, ctypes.c_uint32) for n in "xyz"]
+
+
+class KernelNode(ctypes.Structure):  # hipKernelNodeParams
+    _fields_ = [("block", Dim3), ("extra", ctypes.c_void_p), ("func", ctypes.c_void_p), ("grid", Dim3),
+                ("params", ctypes.c_void_p), ("shared", ctypes.c_uint32)]
+
+
+def grids_of(call):
+    """The grids of the kernels that ``call`` records into a graph."""
     call()
     graph = torch.cuda.CUDAGraph(keep_graph=True)
     torch.cuda.synchronize()
@@ -56,9 +65,15 @@ def kernels_of(call):
         call()
     with open("/proc/self/maps") as f:  # the runtime that torch loaded
         hip = ctypes.CDLL(next(line.split()[-1] for line in f if "libamdhip64.so" in line))
-    count = ctypes.c_size_t()
-    assert hip.hipGraphGetNodes(ctypes.c_void_p(graph.raw_cuda_graph()), None, ctypes.byref(count)) == 0
-    return count.value
+    count, raw = ctypes.c_size_t(), ctypes.c_void_p(graph.raw_cuda_graph())
+    assert hip.hipGraphGetNodes(raw, None, ctypes.byref(count)) == 0
+    nodes, grids = (ctypes.c_void_p * count.value)(), []
+    assert hip.hipGraphGetNodes(raw, nodes, ctypes.byref(count)) == 0
+    for node in nodes:
+        k = KernelNode()
+        assert hip.hipGraphKernelNodeGetParams(ctypes.c_void_p(node), ctypes.byref(k)) == 0
+        grids.append((k.grid.x, k.grid.y, k.grid.z))
+    return grids
 
 
 def chunk_args(n, t, hv):
@@ -75,8 +90,8 @@ def chunk_args(n, t, hv):
     (33, 4, 300, 3), (33, 4, 1300, 11), (39, 4, 450, 4), (48, 2, 200, 4), (1, 4, 5120, 1), (1, 4, 5121, 2)])
 def test_segments_of_dense_batches(n, hv, t, segments):
     q, k, v, g, beta, h0 = chunk_args(n, t, hv)
-    assert kernels_of(lambda: chunk_gated_delta_rule(q, k, v, g, beta, initial_state=h0, output_final_state=True,
-                                                     use_qk_l2norm_in_kernel=True)) == 2 * segments
+    assert len(grids_of(lambda: chunk_gated_delta_rule(q, k, v, g, beta, initial_state=h0, output_final_state=True,
+                                                       use_qk_l2norm_in_kernel=True))) == 2 * segments
 
 
 def test_a_workspace_of_64_chunks_still_serves():
@@ -99,6 +114,17 @@ def test_a_workspace_of_64_chunks_still_serves():
 
     assert call(full - 17 * slot) != 0  # 63 slots: refused
     for bytes_, launches in ((full, 6), (full - 15 * slot, 10)):
-        assert kernels_of(lambda: call(bytes_)) == launches
+        assert len(grids_of(lambda: call(bytes_))) == launches
     (o, s), (o2, s2) = out[1], out[3]  # (out[2], out[4]: captured, not run)
     assert torch.equal(o, o2) and torch.equal(s, s2)
+
+
+# channels, type, tokens, tokens per tile
+@pytest.mark.parametrize("c,dt,t,tile", [
+    (2048, FP32, 2048, 8), (2048, FP32, 3600, 16), (2048, FP32, 3906, 16),  # 16 up to 32 million bytes of x
+    (2048, FP32, 3907, 32), (2048, FP32, 4096, 32), (8192, FP32, 1024, 32), (1024, FP32, 4096, 16), (2048, BF16, 4096, 16),
+    (2048, BF16, 4097, 32), (8192, BF16, 1024, 16)])
+def test_conv_tiles(c, dt, t, tile):
+    gen = torch.Generator(device=DEV).manual_seed(t)
+    x, w = torch.randn(t, c, generator=gen, device=DEV).to(dt), torch.randn(c, 4, generator=gen, device=DEV).to(dt)
+    assert grids_of(lambda: causal_conv1d_fn(x, w, None, "silu")) == [((c // 8 + 255) // 256, (t + tile - 1) // tile, 1)]
