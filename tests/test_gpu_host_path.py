@@ -30,21 +30,24 @@ class Declines:
 
 
 class Counts:
-    """The host extension, counting the calls it took."""
+    """The host extension, counting the calls it took and naming them."""
 
     def __init__(self):
-        self.host, self.took = _lib.host(), 0
+        self.host, self.took, self.names = _lib.host(), 0, set()
 
     def __getattr__(self, name):
         def call(*a):
             r = getattr(self.host, name)(*a)
             self.took += r is not None
+            if r is not None:
+                self.names.add(name)
             return r
         return call
 
 
-def both(monkeypatch, make, call, native=True):
-    """call(make()) natively and the general way: the same bits; whether the native path took it."""
+def both(monkeypatch, make, call, native=True, names=None):
+    """call(make()) natively and the general way: the same bits; whether the native path took it (and, with
+    ``names``, which of its functions did)."""
     outs = []
     for host in (Counts(), Declines()):
         monkeypatch.setattr(_lib, "host", lambda h=host: h)
@@ -53,6 +56,7 @@ def both(monkeypatch, make, call, native=True):
         outs.append([x for x in (r if isinstance(r, tuple) else (r,)) if x is not None] + [a.get("pool")])
         if isinstance(host, Counts):
             assert (host.took > 0) == native
+            assert names is None or host.names == names
     monkeypatch.undo()
     for x, y in zip(*outs):
         if x is not None:
@@ -167,4 +171,6 @@ def test_layer_on_pools(monkeypatch, rows, prefill, t):
         with torch.no_grad():
             y = gated_delta_net_forward(layer, a["x"], cache_params=types.SimpleNamespace(gdn_slot_pools=a["pools"]))
         return y, a["pools"].layer(0)[0]
-    both(monkeypatch, make, call)
+    # (the fixture layer's 4 heads: its b and a stay modules in longer steps)
+    names = {"in_proj", "core_decode", "out_proj"} if t == 1 else {"conv", "chunk" if t > 16 else "recurrent", "rms_norm"}
+    both(monkeypatch, make, call, names=names)

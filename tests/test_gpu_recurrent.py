@@ -340,6 +340,33 @@ def test_token_blocks_match_oracle(b, t, dt, kd, vd):
     assert gdn.state_rel_err(np64(s2), np64(s)) <= 1e-5
 
 
+@pytest.mark.parametrize("b,t,dt,strided", [(1, 5, torch.float32, False), (2, 33, torch.bfloat16, True),
+                                            (3, 65, torch.float32, True), (8, 16, torch.bfloat16, True)])
+def test_token_blocks_with_gates_from_the_projections(b, t, dt, strided):
+    """Gates formed in the token-block kernel from a and b (fp32 or bf16; contiguous, or the columns of one
+    wider projection, read at its token stride), softplus past its threshold among them."""
+    from engine.kernels import fused_recurrent_gated_delta_rule_from_projections
+    hk, hv = 2, 4
+    gen = torch.Generator().manual_seed(10 * b + t)
+    q, k = (torch.randn(b, t, hk, 128, generator=gen).to(dt) for _ in range(2))
+    v = torch.randn(b, t, hv, 128, generator=gen).to(dt)
+    ab = (torch.randn(b, t, 5 * hv, generator=gen) * 3).to(dt)
+    ab[0, -1, hv] = 30.0
+    A_log, dt_bias = torch.linspace(-1, 1, hv), torch.linspace(-1, 1, hv)
+    h0 = torch.randn(b, hv, 128, 128, generator=gen) * 0.1
+    g, beta = gdn.gdn_gates(np64(ab[..., hv:2 * hv]), np64(ab[..., 3 * hv:4 * hv]), np64(A_log), np64(dt_bias))
+    o_ref, s_ref = gdn.recurrent_gated_delta_rule(np64(q), np64(k), np64(v), g, beta, initial_state=h0.numpy())
+    x = ab.to(DEV)
+    a_, b_ = x[..., hv:2 * hv], x[..., 3 * hv:4 * hv]
+    if not strided:
+        a_, b_ = a_.contiguous(), b_.contiguous()
+    o, s = fused_recurrent_gated_delta_rule_from_projections(*cuda(q, k, v), a_, b_, *cuda(A_log, dt_bias),
+                                                             initial_state=h0.to(DEV), output_final_state=True)
+    # fp32 gates of the device's exp and log1p (a few ulp) in an fp32 recurrence of t tokens: far under 1e-5
+    assert np.abs(np64(o) - o_ref).max() <= (1e-4 if dt == torch.float32 else O_TOL_BF16)
+    assert gdn.state_rel_err(np64(s), s_ref) <= 1e-5
+
+
 def test_token_blocks_packed_sequences_on_a_pool():
     """Packed sequences (empty, one token, odd, longer than a block) on a slot pool in place with a repeated
     and a negative id: against one call per sequence's oracle; unowned slots keep their bits."""
