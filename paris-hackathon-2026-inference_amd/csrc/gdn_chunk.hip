@@ -38,8 +38,9 @@
 //                       with buffer_load ... lds.
 //   chunk_scan_cols_kernel  (more pairs) the same with 32 or 64 state columns
 //                       per workgroup, 16 to a compute wave.
-// Inputs longer than one segment (64 chunks) run prep / scan per segment,
-// one segment after the other on the caller's stream.
+// Inputs of more than 80 chunks run prep / scan per segment (64 chunks; of
+// several equal sequences the same window of each), one segment after the
+// other on the caller's stream.
 // Precision (checked against an fp64 restatement at T=4096): the state is fed
 // to MFMA as bf16, U stays fp32 (it initialises the V' accumulator), the state
 // increment K^T V'' uses V'' split into bf16 hi + lo.
@@ -751,7 +752,7 @@ __device__ __forceinline__ RowSrc row_src(const ChunkArgs &a, const ScanRange &s
 
 // Loader ld's copies [i0, i1) of one chunk into stage st (1 KiB each, lane l's
 // 16 bytes at 16 l; a raw row block i holds rows 4i .. 4i + 3, LDS segment ps
-// of a row holding its logical segment ps ^ (row & 15), the nsw layout).
+// of a row holding its logical segment ps ^ row_swizzle(row), the nsw layout).
 template <int LD>
 __device__ __forceinline__ void stage_copy(u32x4 *st, const RowSrc &r, const ChunkArgs &a, int ct, int i0, int i1,
                                            int lane) {
@@ -1947,15 +1948,15 @@ __global__ __launch_bounds__(64 * LOC_WAVES) void chunk_local_kernel(ChunkArgs a
 
 
 // Chunks per prep + scan segment: one prep launch produces a segment's
-// operands (about 2.3 MiB per chunk at 32 v-heads: 146 MiB for 64 chunks,
-// which stay in the 256 MB Infinity Cache until the scan reads them) and one
-// scan launch consumes them; longer inputs run segment after segment on the
-// caller's stream.  Measured (T = 16384 / 65536 / configuration 3): serial
-// 64-chunk segments 478 us / 1.78 ms / 431 us; 96, 128 and 512 chunks, whose
-// operands spill to HBM, 532-560 us / 2.0-2.2 ms / 490-518 us; the next
-// segment's prep on a second stream beside the scan 700 us / 3.1 ms (the two
-// kernels cannot share a CU -- the scan holds 138 KiB of LDS -- so the prep
-// takes CUs from the scan's chain).
+// operands (57 KiB per chunk and v-head, 1.8 MiB per chunk at 32 v-heads:
+// 114 MiB for 64 chunks, which stay in the 256 MB Infinity Cache until the scan
+// reads them) and one scan launch consumes them; longer inputs run segment
+// after segment on the caller's stream.  Measured, T = 6144 / 16384 / 65536:
+// serial 64-chunk segments 150 / 376 us / 1.51 ms; 96 chunks 196 / 482 us /
+// 2.05 ms, 128 chunks 196 / 525 us / 2.07 ms, whose operands spill to HBM.  The
+// next segment's prep on a second stream beside the scan took half as long
+// again (the two kernels cannot share a CU -- the scan holds 132 KiB of LDS --
+// so the prep takes CUs from the scan's chain).
 constexpr int SEG_CHUNKS = 64;
 // ... but a call of up to this many chunks is one segment: the few chunks of
 // a second one would cost a prep and a scan launch of their own, latency-bound
@@ -1966,21 +1967,27 @@ constexpr int SEG_ONE = 80;
 // (sequence, v-head) pairs from which the local kernel runs.  Its time is the
 // longest sequence's chunk count times a chunk step, whatever the batch (up
 // to one workgroup per CU); prep + scan grows with the total chunks.
-// Measured (q/k at 16 heads, Hv = 32): B = 4 x T = 1038 132 (prep + scan)
-// against 139 us, B = 6 x T = 1038 193 against 142, B = 4 x T = 4096 459
-// against 495, B = 2 x T = 4096 242 against 477: the local kernel from 5
-// sequences of 32 v-heads.
+// Measured from graphs (q/k at 16 heads, Hv = 32), prep + scan / local, us, at
+// B = 4 / 5 / 6 / 8 / 9 (two rounds of the CUs) / 12 / 16:
+//   T = 300   35.6/43.0  47.5/43.8  50.9/44.4  64.9/46.2  79.3/79.2  91/84  122/91
+//   T = 1038  94/115  141/119  159/121  211/130  239/229  316/234  435/250
+//   T = 4096  325/398  473/399  545/402  703/457  864/810  1119/829  1555/880
+// (at T = 256 and B = 9 67.8 / 67.6): the local kernel from 5 sequences of 32
+// v-heads.  Of a packed batch only the total is known here; one long sequence
+// among short ones is better on prep + scan (2000 + 5 / 9 x 300 tokens: 96 / 189
+// against 203 / 205 us).
 constexpr int LOC_MIN_PAIRS = 160;
 // Short batches take the local kernel below that as well: one chunk per
 // sequence at any batch, two from LOC_SHORT2_PAIRS pairs, where prep + scan's
 // fixed latency outweighs a chunk step.  The chunk count is exact for a dense
 // batch (no cu_seqlens); with cu_seqlens its bound, the total tokens' chunks
-// (one sequence can hold them all), is used.  Measured from graphs (10 calls per
+// (one sequence can hold them all), is used.  Measured from graphs (6 calls per
 // replay, Hv = 32), local against prep + scan: T = 64 at B = 1 / 2 / 3 / 4
-// 14.1 / 14.5 / 15.3 / 15.9 against 15.3 / 17.1 / 19.5 / 22.0 us; T = 128
-// 20.5 / 21.0 / 21.5 / 21.9 against 16.5 / 19.4 / 23.7 / 26.7; T = 256
-// 33.4-35.5 against 18.6-37.5.  (The workspace size does not depend on
-// this: a local call ignores the workspace it is given.)
+// 15.5 / 16.8 / 17.7 / 18.2 against 16.3 / 17.7 / 19.9 / 20.9 us; T = 128
+// 21.4 / 23.5 / 24.3 / 24.8 against 17.4 / 20.1 / 23.1 / 24.9 (with the column
+// scan the two meet at B = 4); T = 256 33.5-37.3 against 20.2-33.2.  (The
+// workspace size does not depend on this: a local call ignores the workspace
+// it is given.)
 constexpr int LOC_SHORT2_PAIRS = 96;
 // (sequence, v-head) pairs scanned at once up to which chunk_scan_kernel runs:
 // its 8 workgroups per pair then have a CU each.  Up to twice that, 32 state

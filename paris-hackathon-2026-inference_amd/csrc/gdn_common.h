@@ -252,15 +252,6 @@ __device__ __forceinline__ bool repeats_earlier_wave(const int64_t *idx, int64_t
   return false;
 }
 
-// The same test when n differs between lanes (one thread per sequence).
-__device__ __forceinline__ bool repeats_earlier_thread(const int64_t *idx, int64_t n) {
-  if (!idx || n <= 0) return false;
-  const int64_t id = idx[n];
-  bool hit = false;
-  for (int64_t m = 0; m < n; ++m) hit |= idx[m] == id;
-  return hit;
-}
-
 // pool_row with repeated ids mapped to "no row" (n uniform as for repeats_earlier).
 __device__ __forceinline__ int64_t pool_row_first(const int64_t *idx, int64_t n, int64_t rows) {
   const int64_t r = pool_row(idx, n, rows);

@@ -17,12 +17,12 @@ the kernel prologues (``*_from_projections``), q/k passed at their 16 heads
 one-token decode step runs the four input projections and the conv update
 as one HIP kernel (:func:`engine.kernels.in_proj.gdn_in_proj_decode`);
 otherwise qkv, z (and out) are torch matmuls (hipBLASLt), b and a one kernel
-where they have its form (:func:`_gate_projections`), and the conv runs the HIP ``causal_conv1d`` kernels on their output in place.  The cache calls
+where they have its form (:func:`_gate_projections`), and the conv runs the
+HIP ``causal_conv1d`` kernels on their output in place.  The cache calls
 are HF's own, in HF's order, so the layer works with the transformers cache
-unchanged.  With an engine
-slot-pool cache (``cache_params.gdn_slot_pools``, see
-:mod:`engine.runtime.slot_pools`) the kernels address the pools by slot id
-instead.  :func:`install_gdn_layer_patch` swaps it in for the HF layer
+unchanged.  With an engine slot-pool cache (``cache_params.gdn_slot_pools``,
+see :mod:`engine.runtime.slot_pools`) the kernels address the pools by slot
+id instead.  :func:`install_gdn_layer_patch` swaps it in for the HF layer
 classes.
 """
 from __future__ import annotations

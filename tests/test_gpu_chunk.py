@@ -79,11 +79,11 @@ def test_batched_b2_and_gqa_native_equals_repeated():
     assert torch.equal(o2, o) and torch.equal(s2, s)
 
 
-@pytest.mark.parametrize("t", [300, 4200])
+@pytest.mark.parametrize("t", [300, 4200, 5200])
 def test_repeated_qk_single_sequence_equals_native(t):
     """q and k given per v-head (Hk == Hv) as repeat_interleave makes them: the
     prep finds every pair of v-heads repeated and the scan reads one copy of
-    each pair; the results are the GQA call's bits (4200 tokens: two workspace
+    each pair; the results are the GQA call's bits (5200 tokens: two workspace
     segments)."""
     c = configs.config2(seed=11, t=t)
     o, s = run_chunk(c)
@@ -114,8 +114,8 @@ def test_per_v_head_qk_with_partly_repeated_pairs():
 
 
 
-def test_per_v_head_qk_pairs_on_the_persistent_scan():
-    """A batch of three (the persistent scan walks all of their chunks) with
+def test_per_v_head_qk_pairs_on_the_column_scan():
+    """A batch of three (96 pairs: the column scan) with
     q and k given per v-head: pairs repeated in every chunk of every
     sequence, a pair whose odd head differs in one row of the second
     sequence (q of head 7), a pair whose even head differs in one row of the
@@ -215,11 +215,11 @@ def test_state_passing_split_on_gpu():
 
 
 def test_segments_equal_split_calls():
-    """Inputs over 64 chunks run as several prep + scan segments, the state
+    """Inputs over 80 chunks run as several prep + scan segments of 64, the state
     carried between them in fp32: the same bits as splitting the input at a
     segment boundary into two calls threaded through h0 / hT, dense and
-    varlen (both sequences span a segment boundary; several sequences take
-    the persistent scan, which walks them in one workgroup)."""
+    varlen (both sequences span a segment boundary; a segment holds the
+    packed sequences one after the other)."""
     print("chunk segments: dense T=9000", flush=True)
     c = configs.config2(seed=21, t=9000)
     q, k, v, g, beta = (c[x].to(DEV) for x in ("q", "k", "v", "g", "beta"))
@@ -406,7 +406,7 @@ def test_per_pair_kernel_batches_match_the_oracle(b, t, seed):
 
 def test_per_pair_kernel_varlen_on_a_slot_pool():
     """8 packed sequences (256 pairs: the per-pair kernel) of 4,500 (71 chunks,
-    past the two-kernel path's 64-chunk segment), 0, 1, 130, 64, 700, 65 and 17
+    more than one of the two-kernel path's 64-chunk segments), 0, 1, 130, 64, 700, 65 and 17
     tokens on a 12-slot pool, in place, with slot ids [7, 2, 9, 2, -1, 0, 11, 5]
     (row 3 repeats row 1's slot, row 4 has none) and has_initial_state False
     for row 5: rows 3 and 4 start from zero and write nothing, row 5 starts
@@ -469,7 +469,7 @@ def test_per_pair_kernel_many_varlen_sequences(n_seqs):
 @pytest.mark.parametrize("b,t", [(1, 200), (2, 150), (8, 130)])
 def test_fp32_output_through_the_c_abi(b, t):
     """o in fp32 from bf16 q/k/v (the C ABI's o_dtype; the Python entry
-    returns o in q's dtype): the prep + scan path (B = 1), the persistent scan
+    returns o in q's dtype): the prep + scan path (B = 1), the column scan
     (B = 2) and the per-pair kernel (B = 8 x 32 v-heads), against the oracle,
     and rounded to bf16 equal to the bf16-output call."""
     from engine.kernels import _lib
@@ -521,7 +521,7 @@ def test_per_pair_kernel_repeated_qk_equals_native():
 def test_gqa_ratios_other_than_two(hk, hv, b, t):
     """v-heads over k-heads at ratios 4, 8 and 3 and at 16 v-heads, on the
     prep + scan path (B = 1), at B = 8 on the per-pair kernel (256 or 384
-    pairs) or the persistent scan (128 pairs), and the decode recurrence,
+    pairs) or the column scan (128 pairs), and the decode recurrence,
     against the oracle (which repeats the k-heads)."""
     from engine.kernels import fused_recurrent_gated_delta_rule
     gen = torch.Generator().manual_seed(60 + hk + hv + b)

@@ -6,7 +6,7 @@ Hv of 16 or 32 with Hk = Hv, Hv / 2 or Hv / 4, and one of three state
 modes: no initial state; per-sequence initial states with the final states
 returned; a slot pool updated in place with random slot ids (some repeated,
 some negative) and ``has_initial_state``.  Together the cases reach every
-prefill path -- prep + scan, the persistent scan, the per-pair kernel
+prefill path -- prep + scan, the column scan, the per-pair kernel
 (from 160 (sequence, v-head) pairs) and the short batches on it.
 
 Pool semantics checked (the reference cache's gather / scatter,

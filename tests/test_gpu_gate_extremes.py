@@ -9,7 +9,7 @@ beta exactly 0 (no update), exactly 1 and in between.  The chunk form exps
 only non-positive differences of the cumsum, so nothing overflows; entries
 that underflow are zero in fp32 and negligible in fp64 alike.
 
-Paths: one sequence (prep + scan), three packed sequences (persistent scan),
+Paths: one sequence (prep + scan), three sequences (the column scan),
 six packed sequences (the per-pair kernel, 192 (sequence, v-head) pairs).
 Tolerances as everywhere: bf16 outputs max abs error 2e-2, fp32 final
 states relative error 1e-3 norm-wise per (sequence, head); the fp32
@@ -59,7 +59,7 @@ def packed_inputs(lens, seed):
 
 
 @pytest.mark.parametrize("lens,seed", [([300], 1), ([200, 77, 130], 2), ([150, 64, 1, 90, 200, 33], 3)],
-                         ids=["prep_scan", "persistent_scan", "per_pair"])
+                         ids=["prep_scan", "column_scan", "per_pair"])
 def test_chunk_prefill_at_extreme_gates(lens, seed):
     q, k, v, g, beta, h0, cu = packed_inputs(lens, seed)
     o_ref, s_ref = gdn.recurrent_gated_delta_rule_varlen(
@@ -73,7 +73,7 @@ def test_chunk_prefill_at_extreme_gates(lens, seed):
 
 
 @pytest.mark.parametrize("g_val,s_tol", [(-0.05, 1e-3), (0.0, 3e-3)], ids=["slow_decay", "no_decay"])
-@pytest.mark.parametrize("b", [1, 3, 6], ids=["prep_scan", "persistent_scan", "per_pair"])
+@pytest.mark.parametrize("b", [1, 3, 6], ids=["prep_scan", "column_scan", "per_pair"])
 def test_chunk_prefill_with_full_updates(b, g_val, s_tol):
     """beta = 1 on every token and a uniform decay, 300 tokens per sequence.
 

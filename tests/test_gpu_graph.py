@@ -53,7 +53,7 @@ def test_decode_step_graph_replays_match_eager():
         assert torch.equal(pool, pool_eager)
 
 
-@pytest.mark.parametrize("t", [300, 4200])  # one segment; two (64 chunks each)
+@pytest.mark.parametrize("t", [300, 4200, 5200])  # one segment (up to 80 chunks); two of up to 64
 def test_chunk_prefill_graph_replays_match_eager(t):
     c = configs.config2(seed=12, t=t)
     q, k, v, g, beta = (c[x].to(DEV) for x in ("q", "k", "v", "g", "beta"))
@@ -80,7 +80,7 @@ def test_chunk_prefill_graph_replays_match_eager(t):
 def test_varlen_prefill_graph_replays_match_eager(lens):
     """Packed sequences from a graph: configuration 3's lengths (512 pairs:
     the per-pair kernel, its workgroups ranking the lengths in the kernel) and
-    three sequences with an empty one (the persistent scan, with the chunk
+    three sequences with an empty one (the column scan, with the chunk
     table built on the device)."""
     import numpy as np
     cu = torch.tensor(np.concatenate([[0], np.cumsum(lens)]), dtype=torch.int32, device=DEV)
