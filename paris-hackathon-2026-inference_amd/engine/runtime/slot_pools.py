@@ -71,6 +71,7 @@ class GDNSlotPools:
         self._pad = torch.full((), GDN_PAD_SLOT, dtype=torch.int64, device=self.device)
         self._has_state = torch.zeros(self.max_batch, dtype=torch.bool, device=self.device)
         self.batch_size = 0
+        self._rows = (-1, self._slots, self._has_state)  # the buffers' views of the bound rows, and for how many
         self.decode = False
         self.verify_tokens = 0
         self._snap: Dict[int, torch.Tensor] = {}
@@ -126,16 +127,24 @@ class GDNSlotPools:
             self._ensure_verify_buffers(int(verify_tokens))
         self.verify_tokens = int(verify_tokens)
 
+    def _bound(self) -> Tuple[int, torch.Tensor, torch.Tensor]:
+        """The bound rows' views (made once per batch size: a slice costs the
+        interpreter 2 us, in every layer of every step)."""
+        b = self.batch_size
+        if self._rows[0] != b:
+            self._rows = (b, self._slots[:b], self._has_state[:b])
+        return self._rows
+
     def slots(self) -> torch.Tensor:
         """Slot ids of the bound batch (a view of the persistent buffer)."""
-        return self._slots[: self.batch_size]
+        return self._bound()[1]
 
     def has_state(self) -> torch.Tensor:
         """Per row: continue from the slot's state (decode) or start from zero
         (prefill).  A view of a persistent buffer: rows marked in it after
         :meth:`bind` start as marked in every later conv and chunk prefill of
         the bound batch (replays of a captured one included)."""
-        return self._has_state[: self.batch_size]
+        return self._bound()[2]
 
     def read_slots(self) -> torch.Tensor:
         """Slot ids the bound batch's rows start from, by :meth:`has_state`

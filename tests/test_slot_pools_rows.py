@@ -43,6 +43,15 @@ def test_marked_rows_of_a_prefill_continue_from_their_slots():
     assert p.read_slots().tolist() == [PAD, 2]
 
 
+def test_rows_follow_the_batch_size():
+    p = pools()
+    assert p.slots().tolist() == [] and p.read_slots().tolist() == []
+    for ids in ([1, 2, 3], [4], [5, 0, 2], [3, 1, 0]):
+        p.bind(torch.tensor(ids), is_prefill=False)
+        assert p.slots().tolist() == ids and p.has_state().tolist() == [True] * len(ids)
+        assert p.slots().data_ptr() == p._slots.data_ptr() and p.has_state().data_ptr() == p._has_state.data_ptr()
+
+
 @pytest.mark.parametrize("inference", [False, True])
 def test_marks_count_in_inference_mode(inference):
     with torch.inference_mode(inference):
