@@ -9,8 +9,8 @@
 // (16 bytes per lane), and the waves' partial products meet in LDS and are
 // added in wave order, in fp32, and rounded once.  Bound: the bytes a CU
 // brings in (64 CT KiB of weights, from L2, and 64 RT KiB of x).  A whole layer
-// prefill, eager, 1 x 20 / 1 x 500 / 1 x 2000 / 1 x 4096 tokens 156 / 159 / 231 /
-// 387 -> 118 / 121 / 216 / 375 us.
+// prefill, eager, 1 x 20 / 1 x 500 / 1 x 2000 / 1 x 4096 tokens with the modules and
+// with this 165 / 170 / 238 / 399 and 124 / 127 / 226 / 389 us.
 #include "gdn_common.h"
 #include "gdn_gate_proj.h"
 
@@ -101,7 +101,8 @@ __global__ __launch_bounds__(64 * GP_WAVES) __attribute__((amdgpu_waves_per_eu(2
 // library products: 1 / 333 / 1,000 rows 4.4 / 6.2 / 6.6 against 11.6 / 12.2 /
 // 12.3 us (all 64 columns to a workgroup 9.6 / 11.1 / 11.4); 2,000 rows 8.4
 // against 14.7 (11.5); 4,096 12.0 / 15.8; 8,192 14.0 / 18.4; 16,384 18.6 / 26.6;
-// 65,536 79 / 111.
+// 65,536 79 / 111.  K = 1024 and n = 16 take less of both (1 / 1,000 / 8,192 rows, K = 1024,
+// n = 16: 3.4 / 4.6 / 6.8 against 8.3 / 9.2 / 12.2).
 constexpr int GP_CUS = 256;
 
 template <int KS>
